@@ -53,6 +53,7 @@
 #include <chrono>
 #include <cmath>
 #include <numeric>
+#include <type_traits>
 #include <vector>
 
 #include "cvs_internal.hpp"
@@ -222,19 +223,37 @@ __global__ __launch_bounds__(256) void nearest_centre_kernel(const float* __rest
 }
 
 // Centre k = (row-order sum of its members) * (1 / count); zero when empty
-// (src/metal_context.mm:421-434).
-__global__ __launch_bounds__(256) void centre_sum_kernel(const float* __restrict__ rows, int dp,
-                                                         const uint32_t* __restrict__ members,
-                                                         const int64_t* __restrict__ starts,
-                                                         float* __restrict__ cent) {
-  const int k = blockIdx.x;
+// (src/metal_context.mm:421-434).  One wave per centre and 64 columns: the
+// sum's order is fixed, so its additions are a chain; what took the time was
+// each one's load waiting behind the one before (519 us at n = 60,000,
+// d = 384, 244 centres).  A lane holds one member id of each 64, and the 32
+// row loads of a batch are issued before the first is added (36 us).
+__global__ __launch_bounds__(64) void centre_sum_kernel(const float* __restrict__ rows, int dp,
+                                                        const uint32_t* __restrict__ members,
+                                                        const int64_t* __restrict__ starts,
+                                                        float* __restrict__ cent) {
+  constexpr int kBatch = 32;
+  const int k = blockIdx.x, lane = threadIdx.x;
+  const int c = int(blockIdx.y) * 64 + lane;  // dp is a multiple of 64
   const int64_t b = starts[k], e = starts[k + 1];
-  for (int c = threadIdx.x; c < dp; c += blockDim.x) {
-    float s = 0.f;
-    for (int64_t i = b; i < e; ++i) s += rows[int64_t(members[i]) * dp + c];
-    if (e > b) s *= 1.0f / float(e - b);
-    cent[int64_t(k) * dp + c] = s;
+  float s = 0.f;
+  for (int64_t i0 = b; i0 < e; i0 += 64) {
+    const int cnt = int(e - i0 < 64 ? e - i0 : 64);
+    const uint32_t id = members[i0 + (lane < cnt ? lane : 0)];
+#pragma unroll
+    for (int h = 0; h < 64; h += kBatch) {
+      if (h >= cnt) break;
+      float v[kBatch];
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j)
+        v[j] = rows[int64_t(uint32_t(__builtin_amdgcn_readlane(int(id), h + j))) * dp + c];
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j)
+        if (h + j < cnt) s += v[j];
+    }
   }
+  if (e > b) s *= 1.0f / float(e - b);
+  cent[int64_t(k) * dp + c] = s;
 }
 
 // The 3 (p) nearest other centres of each centre from the full table, by
@@ -361,110 +380,232 @@ __global__ __launch_bounds__(256) void group_topk_kernel(const float* __restrict
 // as at the start of the iteration, `prev`) takes the g nearest of itself
 // and every neighbour of its neighbours other than u, distances summed over
 // the padded row (float4 columns tp + 16 j per lane of each 16-lane team).
-// One workgroup of 4 waves per node; wave 0 keeps the list; `changed`
-// counts the nodes whose list changed.
+// One workgroup of 4 waves per node; `changed` counts the nodes whose list
+// changed.
+//
+// Only pairs that the previous iteration did not evaluate are evaluated.
+// `fresh` marks the entries of each list that entered it in the previous
+// iteration (null in the first one: all of them).  A candidate v reached by
+// u -> w -> v with both edges older was evaluated against u then; it is in
+// the list or its key lies above the list's last one, which only decreases.
+// The exception is an id that left u's list in the previous iteration: its
+// key came from the seeding, whose expanded distance is rounded differently
+// (badly so for rows far from the origin), and the distance here may bring
+// it back.  Such ids (`pprev`, the list before the last, less the list) are
+// put into the hash with a tag, and a stale edge evaluates only a tagged id.
+// Lists are thus the ones that evaluating every pair in every iteration
+// gives.
+//
+// What bounds it: row gathers (1.5 KB a row at d = 384) out of L2.  Nodes
+// run in the order of `order` (cluster by cluster), each XCD on a contiguous
+// run of it, so that concurrent workgroups of an XCD gather the rows of few
+// clusters; 16 neighbours' lists are collected at a time by all waves, and
+// the waves evaluate their share without a barrier, each into a list of its
+// own, filtered by the list's last key.  n = 60,000 d = 384 g = 64, sum of
+// the five iterations: 52.7 ms when wave 0 collected one neighbour at a time
+// and every iteration evaluated every pair, 5.0 ms now (3.2 of it the first).
+constexpr int kHopRound = 16;             // neighbours collected at a time
+constexpr uint32_t kHopTag = 0x80000000u; // hash entry of an id that left the list (ids are below 2^31)
+
+template <int DV>  // float4 columns per lane, at least dv
 __global__ __launch_bounds__(256) void two_hop_kernel(const float4* __restrict__ rows, int dq, int dv, uint32_t n,
-                                                      int g, const uint64_t* __restrict__ prev,
-                                                      uint64_t* __restrict__ next,
+                                                      int g, const uint32_t* __restrict__ order,
+                                                      const uint64_t* __restrict__ prev,
+                                                      const uint64_t* __restrict__ pprev,
+                                                      const uint64_t* __restrict__ fresh,
+                                                      uint64_t* __restrict__ next, uint64_t* __restrict__ fresh_next,
                                                       unsigned int* __restrict__ changed) {
   constexpr int H = 1 << kHopHashBits;
-  constexpr int kMaxDv = 1024 / 64;
-  __shared__ uint32_t s_hash[H];
-  __shared__ uint32_t s_nbr[kMaxG];
-  __shared__ uint32_t s_ids[64];
-  __shared__ float s_dist[64];
-  __shared__ uint64_t s_keys[32];
-  __shared__ uint32_t s_ctl[2];
+  static_assert(H >= 2 * kMaxG * kMaxG && kMaxG % kHopRound == 0, "hash at most about half full");
+  constexpr int U = DV <= 8 ? 2 : 1;  // rows in flight per team
+  __shared__ __attribute__((aligned(16))) uint32_t s_hash[H];
+  __shared__ uint32_t s_ids[kHopRound * kMaxG];
+  __shared__ uint64_t s_keys[4][32];
+  __shared__ uint32_t s_cnt[kMaxG / kHopRound];
+  __shared__ uint32_t s_left;  // ids that left the list in the previous iteration
   const int tid = threadIdx.x, lane = tid & 63;
-  const bool lead = __builtin_amdgcn_readfirstlane(tid >> 6) == 0;
-  const int team = tid >> 4, tp = tid & 15;
-  const uint32_t u = blockIdx.x;
-  for (int i = tid; i < H; i += 256) s_hash[i] = kNoId;
-  float4 qv[kMaxDv];
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int team = lane >> 4, tp = lane & 15;  // team of the wave
+  const uint32_t per = (n + 7u) / 8u;          // nodes per XCD
+  const uint32_t pos = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
+  if (blockIdx.x >= 8u * per || pos >= n) return;
+  const uint32_t u = order[pos];
+
+  // The list, and per neighbour which of its entries to take: all over a
+  // fresh edge, else its fresh ones.
+  uint64_t list = lane < g ? prev[int64_t(u) * g + lane] : kNoKey;
+  const uint32_t my_id = list == kNoKey ? kNoId : uint32_t(list) >> 1;
+  const uint64_t fu = fresh ? fresh[u] : ~0ull;
+  uint64_t take = 0;
+  if (my_id != kNoId) take = (!fresh || ((fu >> lane) & 1ull)) ? ~0ull : fresh[my_id];
+  const uint64_t active = __ballot(take != 0);
+  if (active == 0) {  // same for every wave: no pair is new (and no id left the list)
+    if (wave == 0) {
+      if (lane < g) next[int64_t(u) * g + lane] = list;
+      if (lane == 0) fresh_next[u] = 0;
+    }
+    return;
+  }
+  for (int i = tid; i < H / 4; i += 256)
+    reinterpret_cast<uint4*>(s_hash)[i] = uint4{kNoId, kNoId, kNoId, kNoId};
+  if (tid < kMaxG / kHopRound) s_cnt[tid] = 0;
+  float4 qv[DV];
 #pragma unroll
-  for (int j = 0; j < kMaxDv; ++j)
+  for (int j = 0; j < DV; ++j)
     if (j < dv) qv[j] = rows[int64_t(u) * dq + tp + 16 * j];
-  uint64_t list = kNoKey;
   __syncthreads();
-  auto hash_insert = [&](uint32_t id) -> bool {
-    uint32_t h = (id * 0x9E3779B1u) >> (32 - kHopHashBits);
+  auto slot_of = [](uint32_t id) -> uint32_t { return (id * 0x9E3779B1u) >> (32 - kHopHashBits); };
+  // Claims `id` for evaluation: inserts it, or clears its tag.
+  auto claim = [&](uint32_t id) -> bool {
+    uint32_t h = slot_of(id);
     for (;;) {
       const uint32_t old = atomicCAS(&s_hash[h], kNoId, id);
       if (old == kNoId) return true;
       if (old == id) return false;
+      if (old == (id | kHopTag)) return atomicCAS(&s_hash[h], old, id) == old;
       h = (h + 1u) & uint32_t(H - 1);
     }
   };
-  if (lead) {
-    list = lane < g ? prev[int64_t(u) * g + lane] : kNoKey;
-    const uint32_t id = list == kNoKey ? kNoId : uint32_t(list) >> 1;
-    s_nbr[lane] = id;
-    if (id != kNoId) hash_insert(id);
-    if (lane == 0) hash_insert(u);
-  }
-  const uint64_t start_list = list;
-  __syncthreads();
-  int phase = 0;
-  for (int j = 0; j < g; ++j) {
-    const uint32_t nb = s_nbr[j];
-    if (nb == kNoId) continue;
-    uint32_t* const s_nf = s_ctl + phase;
-    phase ^= 1;
-    if (lead) {
-      uint32_t id = kNoId;
-      if (lane < g) {
-        const uint64_t k2 = prev[int64_t(nb) * g + lane];
-        if (k2 != kNoKey) id = uint32_t(k2) >> 1;
-      }
-      const bool fresh = id < n && hash_insert(id);
-      const uint64_t m = __ballot(fresh);
-      if (fresh) s_ids[mbcnt(m)] = id;
-      if (lane == 0) *s_nf = uint32_t(popc(m));
+  // Claims `id` only if it is there with its tag (inserts nothing).
+  auto claim_tagged = [&](uint32_t id) -> bool {
+    uint32_t h = slot_of(id);
+    for (;;) {
+      const uint32_t old = atomicAdd(&s_hash[h], 0u);
+      if (old == kNoId || old == id) return false;
+      if (old == (id | kHopTag)) return atomicCAS(&s_hash[h], old, id) == old;
+      h = (h + 1u) & uint32_t(H - 1);
     }
-    __syncthreads();
-    const int nf = int(*s_nf);
-    if (nf == 0) continue;
-    for (int r0 = 0; r0 < nf; r0 += 16) {
-      const int r = r0 + team;
-      const bool ok = r < nf;
-      const float4* row = rows + int64_t(s_ids[ok ? r : 0]) * dq + tp;
-      float4 x[kMaxDv];
-#pragma unroll
-      for (int jj = 0; jj < kMaxDv; ++jj)
-        if (jj < dv) x[jj] = row[16 * jj];
-      float acc = 0.f;
-#pragma unroll
-      for (int jj = 0; jj < kMaxDv; ++jj) {
-        if (jj < dv) {
-          const float dx = qv[jj].x - x[jj].x, dy = qv[jj].y - x[jj].y;
-          const float dz = qv[jj].z - x[jj].z, dw = qv[jj].w - x[jj].w;
-          acc += (dx * dx + dy * dy) + (dz * dz + dw * dw);
+  };
+  if (wave == 0) {
+    if (my_id != kNoId) claim(my_id);
+    if (lane == 0) claim(u);
+    bool left = false;
+    if (pprev && fu != 0) {  // an id leaves only when another enters
+      const uint64_t k0 = lane < g ? pprev[int64_t(u) * g + lane] : kNoKey;
+      if (k0 != kNoKey) {
+        const uint32_t id = uint32_t(k0) >> 1;
+        uint32_t h = slot_of(id);
+        for (;;) {
+          const uint32_t old = atomicCAS(&s_hash[h], kNoId, id | kHopTag);
+          left = old == kNoId;
+          if (left || old == id) break;
+          h = (h + 1u) & uint32_t(H - 1);
         }
       }
-      acc += xor_lanes_f(acc, 8);
-      acc += xor_lanes_f(acc, 4);
-      acc += xor_lanes_f(acc, 2);
-      acc += xor_lanes_f(acc, 1);
-      if (ok && tp == 0) s_dist[r] = acc;
+    }
+    const bool any = __ballot(left) != 0;
+    if (lane == 0) s_left = any ? 1u : 0u;
+  }
+  const uint64_t bound0 = shfl_u64(list, g - 1);
+  if (wave != 0) list = kNoKey;
+  __syncthreads();
+  const bool left_any = s_left != 0;
+
+  for (int j0 = 0; j0 < g; j0 += kHopRound) {
+    // Collect: this wave's four neighbours of the round, their lists requested together.
+    constexpr int NW = kHopRound / 4;
+    uint64_t key[NW], sel[NW];
+#pragma unroll
+    for (int t = 0; t < NW; ++t) {
+      const int j = j0 + wave + 4 * t;
+      const uint32_t nb = uint32_t(__builtin_amdgcn_readlane(int(my_id), j));
+      const uint32_t lo = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(take)), j));
+      const uint32_t hi = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(take >> 32)), j));
+      sel[t] = (uint64_t(hi) << 32) | lo;
+      const bool want = j < g && nb != kNoId && (left_any || sel[t] != 0);
+      key[t] = kNoKey;
+      if (want && lane < g) key[t] = prev[int64_t(nb) * g + lane];
+    }
+#pragma unroll
+    for (int t = 0; t < NW; ++t) {
+      const uint32_t id = uint32_t(key[t]) >> 1;
+      bool ok = false;
+      if (key[t] != kNoKey && id < n) {
+        if ((sel[t] >> lane) & 1ull)
+          ok = claim(id);
+        else if (left_any)
+          ok = claim_tagged(id);
+      }
+      const uint64_t m = __ballot(ok);
+      if (m == 0) continue;
+      uint32_t base = 0;
+      if (lane == 0) base = atomicAdd(&s_cnt[j0 / kHopRound], uint32_t(popc(m)));
+      base = uint32_t(__builtin_amdgcn_readfirstlane(int(base)));
+      if (ok) s_ids[base + mbcnt(m)] = id;
     }
     __syncthreads();
-    if (lead) {
-      // Candidates at or above the list's g-th key cannot enter it (ids
-      // are unique here): no sort and merge when none is below it.
-      uint64_t key = lane < nf ? (uint64_t(ord_f32(s_dist[lane])) << 32) | (uint64_t(s_ids[lane]) << 1) : kNoKey;
-      const uint32_t glo = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(list)), g - 1));
-      const uint32_t ghi = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(list >> 32)), g - 1));
-      if (sort_below(key, (uint64_t(ghi) << 32) | glo, kNoKey, s_keys) > 0) {
+    const int nf = __builtin_amdgcn_readfirstlane(int(s_cnt[j0 / kHopRound]));
+    if (nf == 0) continue;  // a count of its own per round: nothing of this round is read below
+    // Evaluate: this wave's share, 64 rows at a time; row 4 i + team of a
+    // batch belongs to lane i of the team.
+    const int share = (nf + 3) / 4;
+    const int end = min(nf, share * (wave + 1));
+    for (int b = share * wave; b < end; b += 64) {
+      const int cnt = min(64, end - b);
+      float dist = 0.f;
+      for (int i = 0; 4 * i < cnt; i += U) {
+        float4 x[U][DV];
+#pragma unroll
+        for (int uu = 0; uu < U; ++uu) {
+          const int r = 4 * (i + uu) + team;
+          const float4* row = rows + int64_t(s_ids[b + (r < cnt ? r : 0)]) * dq + tp;
+#pragma unroll
+          for (int jj = 0; jj < DV; ++jj)
+            if (jj < dv) x[uu][jj] = row[16 * jj];
+        }
+#pragma unroll
+        for (int uu = 0; uu < U; ++uu) {
+          float acc = 0.f;
+#pragma unroll
+          for (int jj = 0; jj < DV; ++jj) {
+            if (jj < dv) {
+              const float dx = qv[jj].x - x[uu][jj].x, dy = qv[jj].y - x[uu][jj].y;
+              const float dz = qv[jj].z - x[uu][jj].z, dw = qv[jj].w - x[uu][jj].w;
+              acc += (dx * dx + dy * dy) + (dz * dz + dw * dw);
+            }
+          }
+          acc += xor_lanes_f(acc, 8);
+          acc += xor_lanes_f(acc, 4);
+          acc += xor_lanes_f(acc, 2);
+          acc += xor_lanes_f(acc, 1);
+          if (tp == i + uu) dist = acc;
+        }
+      }
+      // Candidates at or above the g-th key cannot enter the list (ids are
+      // unique here); bit 0 marks the ones that do.
+      const int mine = 4 * tp + team;
+      uint64_t ck = mine < cnt ? (uint64_t(ord_f32(dist)) << 32) | (uint64_t(s_ids[b + mine]) << 1) | 1ull : kNoKey;
+      const uint64_t gth = shfl_u64(list, g - 1);
+      if (sort_below(ck, gth < bound0 ? gth : bound0, kNoKey, s_keys[wave]) > 0) {
         uint64_t l[1] = {list};
-        wave_merge<1>(l, key);
+        wave_merge<1>(l, ck);
         list = lane < g ? l[0] : kNoKey;
       }
     }
+    __syncthreads();
   }
-  if (lead) {
-    if (lane < g) next[int64_t(u) * g + lane] = list;
-    const bool diff = __ballot(list != start_list) != 0;
-    if (diff && lane == 0) atomicAdd(changed, 1u);
+
+  // Merge the waves' lists (through the hash, which is done with).
+  __syncthreads();
+  uint64_t* s_list = reinterpret_cast<uint64_t*>(s_hash);
+  if (wave != 0) s_list[(wave - 1) * 64 + lane] = list;
+  __syncthreads();
+  if (wave == 0) {
+#pragma unroll
+    for (int w = 0; w < 3; ++w) {
+      const uint64_t c = s_list[w * 64 + lane];
+      if (__ballot(c != kNoKey) == 0) continue;
+      uint64_t l[1] = {list};
+      wave_merge<1>(l, c);
+      list = lane < g ? l[0] : kNoKey;
+    }
+    const bool entered = list != kNoKey && (list & 1ull);
+    const uint64_t m = __ballot(entered);
+    if (lane < g) next[int64_t(u) * g + lane] = entered ? list & ~1ull : list;
+    if (lane == 0) {
+      fresh_next[u] = m;
+      if (m != 0) atomicAdd(changed, 1u);
+    }
   }
 }
 
@@ -531,6 +672,25 @@ __global__ void gather_rows_kernel(const float* __restrict__ rows, int dp, const
   const int r = blockIdx.x;
   if (r >= count) return;
   for (int c = threadIdx.x; c < dp; c += blockDim.x) out[int64_t(r) * dp + c] = rows[int64_t(ids[r]) * dp + c];
+}
+
+// Launches two_hop_kernel with the smallest row buffer that holds dp columns.
+void launch_two_hop(hipStream_t s, const float* rows, int dp, uint32_t n, int g, const uint32_t* order,
+                    const uint64_t* prev, const uint64_t* pprev, const uint64_t* fresh, uint64_t* next,
+                    uint64_t* fresh_next, unsigned int* changed) {
+  const int dv = dp / 64;
+  const dim3 grid(8u * ((n + 7u) / 8u));
+  auto go = [&](auto dv_c) {
+    hipLaunchKernelGGL(two_hop_kernel<decltype(dv_c)::value>, grid, dim3(256), 0, s,
+                       reinterpret_cast<const float4*>(rows), dp / 4, dv, n, g, order, prev, pprev, fresh, next,
+                       fresh_next, changed);
+  };
+  if (dv <= 2) go(std::integral_constant<int, 2>{});
+  else if (dv <= 4) go(std::integral_constant<int, 4>{});
+  else if (dv <= 6) go(std::integral_constant<int, 6>{});
+  else if (dv <= 8) go(std::integral_constant<int, 8>{});
+  else go(std::integral_constant<int, 16>{});
+  after_launch("two_hop_kernel");
 }
 
 double seconds_since(std::chrono::steady_clock::time_point t) {
@@ -671,7 +831,8 @@ void build_reference(cvs_context* ctx, const float* rows_in, int64_t n, int64_t 
     cluster_lists(assign);
     CVS_HIP(hipMemcpyAsync(members_d, members.data(), size_t(n) * sizeof(uint32_t), hipMemcpyHostToDevice, s));
     CVS_HIP(hipMemcpyAsync(starts_d, starts.data(), (size_t(K) + 1) * sizeof(int64_t), hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(centre_sum_kernel, dim3(unsigned(K)), dim3(256), 0, s, rows, dp, members_d, starts_d, cent);
+    hipLaunchKernelGGL(centre_sum_kernel, dim3(unsigned(K), unsigned(dp / 64)), dim3(64), 0, s, rows, dp, members_d,
+                       starts_d, cent);
     after_launch("centre_sum_kernel");
   }
   st.kmeans_iterations = uint32_t(iters);
@@ -757,8 +918,8 @@ void build_reference(cvs_context* ctx, const float* rows_in, int64_t n, int64_t 
         CVS_HIP(hipMemcpyAsync(pmembers_d, pmembers.data(), size_t(n) * sizeof(uint32_t), hipMemcpyHostToDevice, s));
         CVS_HIP(hipMemcpyAsync(pstarts_d, pstarts.data(), (size_t(kPqK) + 1) * sizeof(int64_t),
                                hipMemcpyHostToDevice, s));
-        hipLaunchKernelGGL(centre_sum_kernel, dim3(unsigned(kPqK)), dim3(256), 0, s, sub, kPqDim, pmembers_d,
-                           pstarts_d, ctr);
+        hipLaunchKernelGGL(centre_sum_kernel, dim3(unsigned(kPqK), unsigned(kPqDim / 64)), dim3(64), 0, s, sub, kPqDim,
+                           pmembers_d, pstarts_d, ctr);
         after_launch("centre_sum_kernel");
       }
       assign_step(ctr, code_m);  // the codes (:519-548)
@@ -845,22 +1006,35 @@ void build_reference(cvs_context* ctx, const float* rows_in, int64_t n, int64_t 
   // path (src/cagra.cpp:59).
   const auto t_nd = std::chrono::steady_clock::now();
   {
-    uint64_t* other = mem.alloc<uint64_t>(size_t(n) * g);
-    unsigned int* changed_d = mem.alloc<unsigned int>(1);
-    uint64_t* cur = keys;
+    // Nodes in cluster order (see two_hop_kernel); three lists in turn: the
+    // one before the last, the last, the next.
     const int nd_iters = pq ? 0 : 5;
-    for (int iter = 0; iter < nd_iters; ++iter) {
-      CVS_HIP(hipMemsetAsync(changed_d, 0, sizeof(unsigned int), s));
-      hipLaunchKernelGGL(two_hop_kernel, dim3(unsigned(n)), dim3(256), 0, s, reinterpret_cast<const float4*>(rows),
-                         dp / 4, dp / 64, uint32_t(n), g, static_cast<const uint64_t*>(cur), other, changed_d);
-      after_launch("two_hop_kernel");
-      unsigned int changed = 0;
-      CVS_HIP(hipMemcpyAsync(&changed, changed_d, sizeof(unsigned int), hipMemcpyDeviceToHost, s));
-      CVS_HIP(hipStreamSynchronize(s));
-      std::swap(cur, other);
-      ++st.descent_iterations;
-      st.descent_changed_nodes = changed;
-      if (changed == 0) break;
+    uint64_t* cur = keys;
+    if (nd_iters > 0) {
+      CVS_HIP(hipMemcpyAsync(members_d, members.data(), size_t(n) * sizeof(uint32_t), hipMemcpyHostToDevice, s));
+      uint64_t* out = mem.alloc<uint64_t>(size_t(n) * g);
+      uint64_t* spare = mem.alloc<uint64_t>(size_t(n) * g);
+      uint64_t* before = nullptr;
+      uint64_t* fresh_a = mem.alloc<uint64_t>(size_t(n));
+      uint64_t* fresh_b = mem.alloc<uint64_t>(size_t(n));
+      const uint64_t* fresh_cur = nullptr;
+      unsigned int* changed_d = mem.alloc<unsigned int>(1);
+      for (int iter = 0; iter < nd_iters; ++iter) {
+        CVS_HIP(hipMemsetAsync(changed_d, 0, sizeof(unsigned int), s));
+        launch_two_hop(s, rows, dp, uint32_t(n), g, members_d, cur, before, fresh_cur, out, fresh_a, changed_d);
+        unsigned int changed = 0;
+        CVS_HIP(hipMemcpyAsync(&changed, changed_d, sizeof(unsigned int), hipMemcpyDeviceToHost, s));
+        CVS_HIP(hipStreamSynchronize(s));
+        uint64_t* const reuse = before ? before : spare;
+        before = cur;
+        cur = out;
+        out = reuse;
+        fresh_cur = fresh_a;
+        std::swap(fresh_a, fresh_b);
+        ++st.descent_iterations;
+        st.descent_changed_nodes = changed;
+        if (changed == 0) break;
+      }
     }
     uint32_t* ids = graph_on_device ? out_graph : mem.alloc<uint32_t>(size_t(n) * g);
     const size_t count = size_t(n) * g;

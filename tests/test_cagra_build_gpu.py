@@ -248,6 +248,37 @@ def test_reference_build_matches_oracle(ctx, cvs, oracle, n, d, g):
     assert_recall_not_below(s_gpu, s_ref, gt, 10, f"n={n} search recall on the GPU graph vs the oracle's graph")
 
 
+@pytest.mark.parametrize("n,d,g", [(2500, 16, 64), (2500, 130, 33), (2000, 257, 64), (2501, 384, 16), (2000, 512, 7),
+                                   (1501, 1000, 64)])
+def test_reference_descent_is_closed(ctx, n, d, g):
+    """nn-descent evaluates only pairs that its last iteration did not: once no
+    list changes, no 2-hop candidate may be nearer than a list's last entry.
+    Whole-number rows, so that every fp32 distance is exact and keys are
+    (distance, id); one degree and one dimension per row-buffer size, with
+    part-filled 16-neighbour rounds and a node count that is not a multiple
+    of 8."""
+    rng = np.random.default_rng(n + d + g)
+    base = np.rint(clustered(rng, n, d, centers=6, sigma=0.7) * 4.0).astype(np.float32)
+    graph, st = ctx.cagra_build_reference(base, g, exact_limit=0)
+    check_graph(graph, n, g)
+    assert st["descent_changed_nodes"] == 0 or st["descent_iterations"] == 5
+    x = base.astype(np.int64)
+    sq = (x * x).sum(1)
+    dist = sq[:, None] - 2 * (x @ x.T) + sq[None, :]
+    key = dist * n + np.arange(n)[None, :]
+    own = np.take_along_axis(key, graph.astype(np.int64), 1)
+    assert (np.diff(own, axis=1) > 0).all(), "lists are sorted by (distance, id)"
+    open_nodes = 0
+    for u in range(n):
+        two_hop = np.unique(graph[graph[u]])
+        cand = np.setdiff1d(two_hop, np.append(graph[u], u))
+        open_nodes += int((key[u, cand] < own[u, -1]).any())
+    if st["descent_changed_nodes"] == 0:
+        assert open_nodes == 0
+    else:  # the iteration cap: lists that the last iteration changed may open their neighbours' neighbours
+        assert open_nodes <= st["descent_changed_nodes"] * g
+
+
 @pytest.mark.gpu
 def test_reference_pq_build_matches_oracle(ctx, cvs, oracle):
     """The reference's N > 200,000 build (product-quantised per-cluster
