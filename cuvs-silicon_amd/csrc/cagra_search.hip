@@ -44,6 +44,7 @@
 // with UINT32_MAX / +inf (src/cagra.cpp:240-251).
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "cvs_internal.hpp"
 #include "device_util.hpp"
@@ -126,6 +127,289 @@ __device__ __forceinline__ void merge_into(uint64_t (&top)[E], uint64_t c) {
   }
 }
 
+// The list's last kept key (position itopk - 1; the empty key while the list
+// is not full).
+template <int E>
+__device__ __forceinline__ uint64_t last_key(const uint64_t (&top)[E], int itopk) {
+  const int wpos = itopk - 1;
+  uint64_t worst = kEmptyKey;
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    if (e == (wpos >> 6)) {  // uniform: one slot is read
+      const uint32_t wlo = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(top[e])), wpos & 63));
+      const uint32_t whi = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(top[e] >> 32)), wpos & 63));
+      worst = (uint64_t(whi) << 32) | wlo;
+    }
+  }
+  return worst;
+}
+
+// Inserts one key (uniform over the wave, not in the list) into the sorted
+// list: entries above it move up by one position, the last one falls out.
+// About 10 instructions per slot, where sorting a few candidates and merging
+// them takes over 100 plus 60 per slot.
+template <int E>
+__device__ __forceinline__ void insert_key(uint64_t (&top)[E], uint64_t key) {
+  constexpr int kWaveShr1 = 0x138;  // DPP: lane l takes lane l - 1, lane 0 keeps `old`
+#pragma unroll
+  for (int e = E - 1; e >= 0; --e) {
+    const int lo = int(uint32_t(top[e])), hi = int(uint32_t(top[e] >> 32));
+    int olo = 0, ohi = 0;
+    if (e > 0) {
+      olo = __builtin_amdgcn_readlane(int(uint32_t(top[e - 1])), 63);
+      ohi = __builtin_amdgcn_readlane(int(uint32_t(top[e - 1] >> 32)), 63);
+    }
+    const uint32_t plo = uint32_t(__builtin_amdgcn_update_dpp(olo, lo, kWaveShr1, 0xF, 0xF, false));
+    const uint32_t phi = uint32_t(__builtin_amdgcn_update_dpp(ohi, hi, kWaveShr1, 0xF, 0xF, false));
+    const uint64_t prev = (uint64_t(phi) << 32) | plo;  // 0 before the first entry: below every key
+    top[e] = top[e] < key ? top[e] : (prev < key ? key : prev);
+  }
+}
+
+// Candidate keys (one per lane, the empty key for none) into the list.  A
+// key at or above the list's last one cannot enter it (keys are unique; an
+// unfilled list holds the empty key there), so such candidates are dropped
+// first; a few are inserted one by one, more are compacted (through
+// `scratch`, 32 keys of LDS that only this wave uses here), sorted and
+// merged.  The list is the same either way.
+constexpr int kInsertMax = 6;
+template <int E>
+__device__ __forceinline__ void add_keys(uint64_t (&top)[E], uint64_t key, int itopk, uint64_t* scratch) {
+  const int lane = __lane_id();
+  const uint64_t worst = last_key<E>(top, itopk);
+  uint64_t m = __ballot(key < worst);
+  if (m == 0) return;
+  if (popc(m) <= kInsertMax) {
+    do {
+      const int b = __builtin_ctzll(m);
+      m &= m - 1;
+      const uint32_t lo = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(key)), b));
+      const uint32_t hi = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(key >> 32)), b));
+      insert_key<E>(top, (uint64_t(hi) << 32) | lo);
+    } while (m != 0);
+  } else {
+    (void)sort_below(key, worst, kEmptyKey, scratch);
+    merge_into<E>(top, key);
+  }
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    if (e * 64 + lane >= itopk) top[e] = kEmptyKey;
+}
+
+// A lane's slice of the query and its pieces of a row (d <= 1024).  fp32
+// traversal: float4 columns tp + 16 j of the padded row.  fp16 traversal (and
+// its fp32 re-rank): 8-column pieces tp + 16 j, so that a 16-lane team reads
+// 256 contiguous bytes of an fp16 row (512 of an fp32 row) per piece.  The
+// fp16 traversal keeps its slice of the centred, scaled query in fp16, as the
+// rows are: a piece's distance is four packed differences and four
+// fp32-accumulating dot2s, and the slice takes 32 VGPRs instead of 64.  The
+// traversal's distances only steer the search; the list is re-ranked against
+// the fp32 query and rows at the end.  Query loads are unconditional (column
+// clamped, the value masked by an AND of its bits), so that all are in flight
+// together, and four columns wide where the query's rows are 16-byte aligned.
+__device__ __forceinline__ float masked(float x, bool in) {
+  return __uint_as_float(__float_as_uint(x) & (in ? 0xffffffffu : 0u));
+}
+
+// Sum of the squares of four differences, in one rounding order wherever it
+// is inlined, so that every kernel gives a row the same distance.
+__device__ __forceinline__ float sum_sq4(float x, float y, float z, float w) {
+  return __builtin_fmaf(x, x, __fmul_rn(y, y)) + __builtin_fmaf(z, z, __fmul_rn(w, w));
+}
+
+// Columns c .. c + 3 of a query, zero past d.
+__device__ __forceinline__ float4 query_cols(const SearchArgs& a, const float* qsrc, bool vec, int64_t c) {
+  float4 v;
+  if (vec) {  // d is a multiple of 4: all four columns or none
+    v = *reinterpret_cast<const float4*>(qsrc + (c < a.d ? c : 0));
+    return make_float4(masked(v.x, c < a.d), masked(v.y, c < a.d), masked(v.z, c < a.d), masked(v.w, c < a.d));
+  }
+  const int64_t e = a.d - 1;
+  v = make_float4(qsrc[c < e ? c : e], qsrc[c + 1 < e ? c + 1 : e], qsrc[c + 2 < e ? c + 2 : e],
+                  qsrc[c + 3 < e ? c + 3 : e]);
+  return make_float4(masked(v.x, c < a.d), masked(v.y, c + 1 < a.d), masked(v.z, c + 2 < a.d), masked(v.w, c + 3 < a.d));
+}
+__device__ __forceinline__ bool wide_query(const SearchArgs& a, const float* qsrc) {
+  return (a.d & 3) == 0 && (reinterpret_cast<uintptr_t>(qsrc) & 15) == 0;
+}
+
+template <bool F16>
+struct Slice;
+
+template <>
+struct Slice<false> {
+  using Piece = float4;
+  static constexpr int N = kMaxDv;
+  float4 q[N];
+  __device__ __forceinline__ void load(const SearchArgs& a, const float* qsrc, int tp) {
+    if (wide_query(a, qsrc)) {
+#pragma unroll
+      for (int j = 0; j < N; ++j) q[j] = query_cols(a, qsrc, true, int64_t(tp + 16 * j) * 4);
+    } else {
+#pragma unroll
+      for (int j = 0; j < N; ++j) q[j] = query_cols(a, qsrc, false, int64_t(tp + 16 * j) * 4);
+    }
+  }
+  __device__ __forceinline__ void fetch(const SearchArgs& a, uint32_t rid, int tp, float4 (&x)[N]) const {
+    const float4* row = a.rows + int64_t(rid) * a.dq + tp;
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      if (j < a.dv) x[j] = row[16 * j];
+  }
+  // This lane's part of the squared distance.
+  __device__ __forceinline__ float part(const SearchArgs& a, const float4 (&x)[N]) const {
+    float acc = 0.f;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      if (j < a.dv) {
+        acc = __fadd_rn(acc, sum_sq4(q[j].x - x[j].x, q[j].y - x[j].y, q[j].z - x[j].z, q[j].w - x[j].w));
+      }
+    }
+    return acc;
+  }
+};
+
+template <>
+struct Slice<true> {
+  using Piece = uint4;
+  static constexpr int N = kMaxDv8;
+  half8_t q[N];
+  __device__ __forceinline__ void load(const SearchArgs& a, const float* qsrc, int tp) {
+    if (wide_query(a, qsrc))
+      load_cols(a, qsrc, tp, true);
+    else
+      load_cols(a, qsrc, tp, false);
+  }
+  // Centred and scaled as the traversal copy is (distances in the traversal
+  // are scale^2 times the squared distance), rounded to fp16.  mu holds zeros
+  // past d.
+  __device__ __forceinline__ void load_cols(const SearchArgs& a, const float* qsrc, int tp, bool vec) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const int64_t c = int64_t(tp + 16 * j) * 8;
+      const float4* mu = reinterpret_cast<const float4*>(a.mu + (j < a.dv8 ? c : 0));
+      const float4 x = query_cols(a, qsrc, vec, c), y = query_cols(a, qsrc, vec, c + 4), mx = mu[0], my = mu[1];
+      const float v[8] = {x.x - mx.x, x.y - mx.y, x.z - mx.z, x.w - mx.w, y.x - my.x, y.y - my.y, y.z - my.z, y.w - my.w};
+#pragma unroll
+      for (int t = 0; t < 8; ++t) q[j][t] = _Float16(masked(v[t] * a.scale, c + t < a.d));
+    }
+  }
+  __device__ __forceinline__ void fetch(const SearchArgs& a, uint32_t rid, int tp, uint4 (&x)[N]) const {
+    const uint4* row = a.rows16 + int64_t(rid) * a.dq8 + tp;
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+      if (j < a.dv8) x[j] = row[16 * j];
+  }
+  __device__ __forceinline__ float part(const SearchArgs& a, const uint4 (&x)[N]) const {
+    float acc = 0.f;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      if (j < a.dv8) {
+        const uint4 qw = __builtin_bit_cast(uint4, q[j]);
+        const uint32_t qa[4] = {qw.x, qw.y, qw.z, qw.w}, xa[4] = {x[j].x, x[j].y, x[j].z, x[j].w};
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const half2_t d2 = __builtin_bit_cast(half2_t, qa[t]) - __builtin_bit_cast(half2_t, xa[t]);
+          acc = __builtin_amdgcn_fdot2(d2, d2, acc, false);
+        }
+      }
+    }
+    return acc;
+  }
+};
+
+// Sum over the 16 lanes of a team.
+__device__ __forceinline__ float team_sum(float acc) {
+  acc += xor_lanes_f(acc, 8);
+  acc += xor_lanes_f(acc, 4);
+  acc += xor_lanes_f(acc, 2);
+  acc += xor_lanes_f(acc, 1);
+  return acc;
+}
+
+// Exact part of the squared distance for the re-rank after fp16 traversal
+// (d <= 1024): the fp32 row against the query as given, staged in LDS (zero
+// past d as the rows are).
+__device__ __forceinline__ float exact_part(const SearchArgs& a, const float* s_q, uint32_t rid, int tp) {
+  const float4* row = a.rows + int64_t(rid) * a.dq + 2 * tp;
+  const float4* qq = reinterpret_cast<const float4*>(s_q) + 2 * tp;
+  float acc = 0.f;
+  float4 x[2 * kMaxDv8];
+#pragma unroll
+  for (int j = 0; j < kMaxDv8; ++j) {
+    if (j < a.dv8) {
+      x[2 * j] = row[32 * j];
+      x[2 * j + 1] = row[32 * j + 1];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < kMaxDv8; ++j) {
+    if (j < a.dv8) {
+      const float4 ql = qq[32 * j], qh4 = qq[32 * j + 1];
+      const float4 lo = x[2 * j], hi = x[2 * j + 1];
+      acc = __fadd_rn(acc, sum_sq4(ql.x - lo.x, ql.y - lo.y, ql.z - lo.z, ql.w - lo.w) +
+                               sum_sq4(qh4.x - hi.x, qh4.y - hi.y, qh4.z - hi.z, qh4.w - hi.w));
+    }
+  }
+  return acc;
+}
+
+// Writes a query's results (lead wave): the team's list for the merge of
+// teams, else the k nearest and the counts.
+template <int E>
+__device__ __forceinline__ void write_list(const SearchArgs& a, const uint64_t (&top)[E], int64_t qi, uint32_t evals,
+                                           int it) {
+  const int lane = __lane_id();
+  if (a.team_keys) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int pos = e * 64 + lane;
+      if (pos < a.itopk) a.team_keys[int64_t(blockIdx.x) * a.itopk + pos] = top[e];
+    }
+    return;
+  }
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int pos = e * 64 + lane;
+    if (pos < a.k) {
+      const uint64_t key = top[e];
+      a.out_nbr[qi * a.k + pos] = key == kEmptyKey ? kInvalidId : uint32_t(key) >> 1;
+      a.out_dist[qi * a.k + pos] = key == kEmptyKey ? INFINITY : unord_f32(uint32_t(key >> 32));
+    }
+  }
+  if (a.stats && lane == 0) {
+    a.stats[2 * qi] = evals;
+    a.stats[2 * qi + 1] = uint32_t(it);
+  }
+}
+
+// fp16 traversal: the list's distances are recomputed exactly from the fp32
+// rows (all W waves, 64 entries per round; `exact(id)` sums a row over the
+// calling team) and the list re-sorted, so the output is the exact top-k of
+// the visited rows in the list.
+template <int E, int W, typename Exact>
+__device__ __forceinline__ void rerank_list(uint64_t (&top)[E], bool lead, uint32_t* s_ids, float* s_dist,
+                                            Exact exact) {
+  const int lane = threadIdx.x & 63, team = threadIdx.x >> 4, tp = threadIdx.x & 15;
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    if (lead) s_ids[lane] = top[e] != kEmptyKey ? uint32_t(top[e]) >> 1 : 0u;
+    __syncthreads();
+    for (int r0 = 0; r0 < 64; r0 += 4 * W) {
+      const float acc = exact(s_ids[r0 + team]);
+      if (tp == 0) s_dist[r0 + team] = acc;
+    }
+    __syncthreads();
+    if (lead && top[e] != kEmptyKey) top[e] = (uint64_t(ord_f32(s_dist[lane])) << 32) | (uint64_t(s_ids[lane]) << 1);
+  }
+  if (lead) wave_sort_e<E>(top);
+}
+
+// The query as given into LDS (kBigDim floats, zero past d).
+__device__ __forceinline__ void stage_query(const SearchArgs& a, const float* qsrc, float* s_q, int threads) {
+  for (int i = threadIdx.x; i < kBigDim; i += threads) s_q[i] = masked(qsrc[i < a.d ? i : a.d - 1], i < a.d);
+}
+
 // One workgroup of W waves per query.  Wave 0 (the lead wave) owns the
 // itopk list, the hash inserts, the sort and the merge; all 4W 16-lane teams
 // gather candidate rows, so a chunk of 64 candidates costs ceil(64 / 4W)
@@ -179,43 +463,9 @@ __global__ __launch_bounds__(64 * W, (F16 && W == 2 && !BIG) ? 4 : 1) void cagra
     }
   }
 
-  // Query slice of this lane (d <= 1024).  fp32 traversal: float4 columns tp + 16 j of
-  // the padded row.  fp16 traversal (and its fp32 re-rank): 8-column pieces
-  // tp + 16 j, so that a 16-lane team reads 256 contiguous bytes of an fp16
-  // row (512 of an fp32 row) per piece.  The fp16 traversal keeps its slice
-  // of the centred, scaled query in fp16, as the rows are: a piece's
-  // distance is four packed differences and four fp32-accumulating dot2s,
-  // and the slice takes 32 VGPRs instead of 64.  The traversal's distances
-  // only steer the search; the list is re-ranked against the fp32 query and
-  // rows at the end.
   const float* qsrc = a.queries + qi * a.d;
-  float4 qv[F16 || BIG ? 1 : kMaxDv];
-  half8_t qh[F16 && !BIG ? kMaxDv8 : 1];
-  if constexpr (BIG) {
-  } else if constexpr (!F16) {
-#pragma unroll
-    for (int j = 0; j < kMaxDv; ++j) {
-      float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (j < a.dv) {
-        const int64_t c = int64_t(tp + 16 * j) * 4;
-        if (c + 0 < a.d) t.x = qsrc[c + 0];
-        if (c + 1 < a.d) t.y = qsrc[c + 1];
-        if (c + 2 < a.d) t.z = qsrc[c + 2];
-        if (c + 3 < a.d) t.w = qsrc[c + 3];
-      }
-      qv[j] = t;
-    }
-  } else {
-    // Centred and scaled as the traversal copy is (distances in the
-    // traversal are scale^2 times the squared distance), rounded to fp16.
-#pragma unroll
-    for (int j = 0; j < kMaxDv8; ++j)
-#pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        const int64_t c = int64_t(tp + 16 * j) * 8 + t;
-        qh[j][t] = _Float16((j < a.dv8 && c < a.d) ? (qsrc[c] - a.mu[c]) * a.scale : 0.f);
-      }
-  }
+  Slice<F16> slice;  // d <= 1024
+  if constexpr (!BIG) slice.load(a, qsrc, tp);
 
   // Squared distance of row rid to the query, summed over the 16 lanes of
   // this lane's team: from the traversal copy, or (exact) from the fp32 rows.
@@ -270,69 +520,14 @@ __global__ __launch_bounds__(64 * W, (F16 && W == 2 && !BIG) ? 4 : 1) void cagra
           }
         }
       }
-    } else if constexpr (!F16) {
-      const float4* row = a.rows + int64_t(rid) * a.dq + tp;
-      float4 x[kMaxDv];
-#pragma unroll
-      for (int j = 0; j < kMaxDv; ++j)
-        if (j < a.dv) x[j] = row[16 * j];
-#pragma unroll
-      for (int j = 0; j < kMaxDv; ++j) {
-        if (j < a.dv) {
-          const float dx = qv[j].x - x[j].x, dy = qv[j].y - x[j].y;
-          const float dz = qv[j].z - x[j].z, dw = qv[j].w - x[j].w;
-          acc += (dx * dx + dy * dy) + (dz * dz + dw * dw);
-        }
-      }
-    } else if (!exact) {
-      const uint4* row = a.rows16 + int64_t(rid) * a.dq8 + tp;
-      uint4 x[kMaxDv8];
-#pragma unroll
-      for (int j = 0; j < kMaxDv8; ++j)
-        if (j < a.dv8) x[j] = row[16 * j];
-#pragma unroll
-      for (int j = 0; j < kMaxDv8; ++j) {
-        if (j < a.dv8) {
-          const uint4 qw = __builtin_bit_cast(uint4, qh[j]);
-          const uint32_t qa[4] = {qw.x, qw.y, qw.z, qw.w}, xa[4] = {x[j].x, x[j].y, x[j].z, x[j].w};
-#pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            const half2_t d2 = __builtin_bit_cast(half2_t, qa[t]) - __builtin_bit_cast(half2_t, xa[t]);
-            acc = __builtin_amdgcn_fdot2(d2, d2, acc, false);
-          }
-        }
-      }
+    } else if (F16 && exact) {
+      acc = exact_part(a, s_q, rid, tp);
     } else {
-      // Exact: the fp32 rows against the query as given (staged in LDS, zero
-      // past d as the rows are; this runs once per list entry at the end of
-      // the search).
-      const float4* row = a.rows + int64_t(rid) * a.dq + 2 * tp;
-      const float4* qq = reinterpret_cast<const float4*>(s_q) + 2 * tp;
-      float4 x[2 * kMaxDv8];
-#pragma unroll
-      for (int j = 0; j < kMaxDv8; ++j) {
-        if (j < a.dv8) {
-          x[2 * j] = row[32 * j];
-          x[2 * j + 1] = row[32 * j + 1];
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < kMaxDv8; ++j) {
-        if (j < a.dv8) {
-          const float4 ql = qq[32 * j], qh4 = qq[32 * j + 1];
-          const float qr[8] = {ql.x, ql.y, ql.z, ql.w, qh4.x, qh4.y, qh4.z, qh4.w};
-          const float4 lo = x[2 * j], hi = x[2 * j + 1];
-          const float d0 = qr[0] - lo.x, d1 = qr[1] - lo.y, d2 = qr[2] - lo.z, d3 = qr[3] - lo.w;
-          const float d4 = qr[4] - hi.x, d5 = qr[5] - hi.y, d6 = qr[6] - hi.z, d7 = qr[7] - hi.w;
-          acc += ((d0 * d0 + d1 * d1) + (d2 * d2 + d3 * d3)) + ((d4 * d4 + d5 * d5) + (d6 * d6 + d7 * d7));
-        }
-      }
+      typename Slice<F16>::Piece x[Slice<F16>::N];
+      slice.fetch(a, rid, tp, x);
+      acc = slice.part(a, x);
     }
-    acc += xor_lanes_f(acc, 8);
-    acc += xor_lanes_f(acc, 4);
-    acc += xor_lanes_f(acc, 2);
-    acc += xor_lanes_f(acc, 1);
-    return acc;
+    return team_sum(acc);
   };
 
   uint64_t top[E];  // the list (lead wave)
@@ -406,28 +601,9 @@ __global__ __launch_bounds__(64 * W, (F16 && W == 2 && !BIG) ? 4 : 1) void cagra
     if (lead) {
       uint64_t key =
           lane < nf ? (uint64_t(ord_f32(s_dist[lane])) << 32) | (uint64_t(s_ids[lane]) << 1) : kEmptyKey;
-      // A key at or above the list's itopk-th key cannot enter the list
-      // (keys are unique; an unfilled list holds the empty key there), so
-      // such candidates are dropped first: no sort at all when none is
-      // left, and a few are compacted into the first lanes (through the
-      // id/distance slots, which every wave has finished reading) and
-      // sorted over 16 or 32 lanes.  The merged list is the same.
-      const int wpos = a.itopk - 1;
-      uint64_t worst = kEmptyKey;
-#pragma unroll
-      for (int e = 0; e < E; ++e) {
-        if (e == (wpos >> 6)) {  // uniform: one slot is read
-          const uint32_t wlo = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(top[e])), wpos & 63));
-          const uint32_t whi = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(top[e] >> 32)), wpos & 63));
-          worst = (uint64_t(whi) << 32) | wlo;
-        }
-      }
-      if (sort_below(key, worst, kEmptyKey, reinterpret_cast<uint64_t*>(s_ids)) > 0) {
-        merge_into<E>(top, key);
-#pragma unroll
-        for (int e = 0; e < E; ++e)
-          if (e * 64 + lane >= a.itopk) top[e] = kEmptyKey;
-      }
+      // (The id/distance slots are the scratch: every wave has finished
+      // reading them.)
+      add_keys<E>(top, key, a.itopk, reinterpret_cast<uint64_t*>(s_ids));
     }
     // With one wave, program order alone separates this chunk's LDS reads
     // from the next chunk's writes; with more, the lead wave writes the next
@@ -496,55 +672,504 @@ __global__ __launch_bounds__(64 * W, (F16 && W == 2 && !BIG) ? 4 : 1) void cagra
     }
   }
 
-  // fp16 traversal: the list's distances are recomputed exactly from the
-  // fp32 rows (all teams, 64 entries per round) and the list re-sorted, so
-  // the output is the exact top-k of the visited rows in the list.
   if constexpr (F16) {
-    if constexpr (!BIG) {
-      // The query as given into LDS for the exact distances (the loop's
-      // first barrier publishes it): global loads issued together (column
-      // clamped, value masked by an AND of its bits), where per-element
-      // loads under the column test took one round trip per 8 columns.
-      for (int i = tid; i < kBigDim; i += kThreads) {
-        const float x = qsrc[i < a.d ? i : a.d - 1];
-        s_q[i] = __uint_as_float(__float_as_uint(x) & (i < a.d ? 0xffffffffu : 0u));
-      }
+    if constexpr (!BIG) stage_query(a, qsrc, s_q, kThreads);  // published by the re-rank's first barrier
+    rerank_list<E, W>(top, lead, s_ids, s_dist, [&](uint32_t rid) { return team_dist(rid, true); });
+  }
+  if (lead) write_list<E>(a, top, qi, evals, it);
+}
+
+// Smallest value of the wave, in every lane: v_min_u32 with DPP row shifts
+// and row broadcasts (lanes without a source take the identity).
+__device__ __forceinline__ uint32_t wave_min_u32(uint32_t x) {
+  auto step = [&](auto ctrl, auto rows) {
+    constexpr int kCtrl = decltype(ctrl)::value, kRows = decltype(rows)::value;
+    const uint32_t y = uint32_t(__builtin_amdgcn_update_dpp(-1, int(x), kCtrl, kRows, 0xF, false));
+    x = y < x ? y : x;
+  };
+  using std::integral_constant;
+  step(integral_constant<int, 0x111>{}, integral_constant<int, 0xF>{});  // row_shr:1, 2, 4, 8
+  step(integral_constant<int, 0x112>{}, integral_constant<int, 0xF>{});
+  step(integral_constant<int, 0x114>{}, integral_constant<int, 0xF>{});
+  step(integral_constant<int, 0x118>{}, integral_constant<int, 0xF>{});
+  step(integral_constant<int, 0x142>{}, integral_constant<int, 0xA>{});  // row_bcast:15 into rows 1 and 3
+  step(integral_constant<int, 0x143>{}, integral_constant<int, 0xC>{});  // row_bcast:31 into rows 2 and 3
+  return uint32_t(__builtin_amdgcn_readlane(int(x), 63));
+}
+
+// The itopk list of cagra_ahead_kernel, split so that the steps of one wave
+// take few dependent instructions however long the list is.  A fully sorted
+// list is not needed for the search: the next parent is the smallest
+// unexpanded key, and it is in the list iff fewer than itopk expanded keys lie
+// below it (no other unexpanded key does).
+//  - front: the nearest unexpanded keys, sorted, one per lane.
+//  - buf: keys on their way into `rest` (LDS).  They stay there unsorted until
+//    front is taken anew: by then most of them lie beyond the list.
+//  - rest: the other keys, sorted, at most itopk; bit 0 is set in expanded ones.
+// Every unexpanded key outside front is at or above flim, every one in it
+// below.  Keys at or above `bound`, the last key of a full list, cannot be
+// in it and are dropped; keys beyond the list that are kept are harmless, as
+// the test above rejects them as parents and the list is cut to itopk keys at
+// the end.  One wave uses the pool; every member but front and rest is uniform
+// over it.
+template <int E>
+struct Pool {
+  static constexpr int kFull = 512;              // buf is emptied at this many keys
+  static constexpr int kBuf = kFull + 128 + 16;  // one add, the parents of one step
+  static constexpr int kNear = 65;               // refill: the nearest unexpanded keys and one more
+  static constexpr int kLds = kBuf + kNear + 64 * E;
+  uint64_t front, rest[E];
+  uint64_t bound, flim;
+  int nbuf, expanded, itopk;
+  uint64_t* buf;
+
+  // The seeds go to `rest` (merge_sorted); flim = 0 makes front take them.
+  __device__ __forceinline__ void init(int itopk_, uint64_t* lds) {
+    front = kEmptyKey;
+#pragma unroll
+    for (int e = 0; e < E; ++e) rest[e] = kEmptyKey;
+    bound = kEmptyKey;
+    flim = 0;
+    nbuf = expanded = 0;
+    itopk = itopk_;
+    buf = lds;
+  }
+  // 64 sorted keys into `rest`.
+  __device__ __forceinline__ void merge_sorted(uint64_t key) {
+    const int lane = __lane_id();
+    merge_into<E>(rest, key);
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+      if (e * 64 + lane >= itopk) rest[e] = kEmptyKey;
+  }
+  // The whole list into `rest`: front first, then what of `buf` is still
+  // below the list's last key.
+  __device__ __forceinline__ void collect() {
+    merge_sorted(front);
+    front = kEmptyKey;
+#pragma unroll 1
+    for (int b = 0; b < nbuf; b += 64) {
+      const int i = b + int(__lane_id());
+      add_keys<E>(rest, i < nbuf ? buf[i] : kEmptyKey, itopk, buf + kBuf);
     }
+    nbuf = 0;
+    const uint64_t w = last_key<E>(rest, itopk);
+    bound = w < bound ? w : bound;  // (refill takes keys out of `rest` again)
+  }
+  __device__ __forceinline__ void refill() {
+    const int lane = __lane_id();
+    collect();
+    uint64_t* near = buf + kBuf;
+    uint64_t* kept = near + kNear;
+    int nu = 0, nk = 0;
 #pragma unroll
     for (int e = 0; e < E; ++e) {
-      if (lead) s_ids[lane] = top[e] != kEmptyKey ? uint32_t(top[e]) >> 1 : 0u;
-      __syncthreads();
-      for (int r0 = 0; r0 < 64; r0 += kTeams) {
-        const float acc = team_dist(s_ids[r0 + team], true);
-        if (tp == 0) s_dist[r0 + team] = acc;
-      }
-      __syncthreads();
-      if (lead && top[e] != kEmptyKey) top[e] = (uint64_t(ord_f32(s_dist[lane])) << 32) | (uint64_t(s_ids[lane]) << 1);
+      const bool un = rest[e] != kEmptyKey && (rest[e] & 1ull) == 0;
+      const uint64_t m = __ballot(un);
+      const int r = nu + mbcnt(m);
+      if (un && r < kNear) near[r] = rest[e];
+      const bool keep = rest[e] != kEmptyKey && !(un && r < 64);
+      const uint64_t mk = __ballot(keep);
+      if (keep) kept[nk + mbcnt(mk)] = rest[e];
+      nu += popc(m);
+      nk += popc(mk);
     }
-    if (lead) wave_sort_e<E>(top);
+    front = lane < nu ? near[lane] : kEmptyKey;
+    const uint64_t next = near[nu > 64 ? 64 : 0];
+    flim = nu > 64 ? (uint64_t(uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(next >> 32))))) << 32) |
+                         uint32_t(__builtin_amdgcn_readfirstlane(int(uint32_t(next))))
+                   : kEmptyKey;
+#pragma unroll
+    for (int e = 0; e < E; ++e) rest[e] = e * 64 + lane < nk ? kept[e * 64 + lane] : kEmptyKey;
+  }
+  // Number of entries in `front`, at least `want` if there are as many
+  // unexpanded keys at all.
+  __device__ __forceinline__ int ready(int want) {
+    int c = popc(__ballot(front != kEmptyKey));
+    if ((c < want && flim != kEmptyKey) || nbuf >= kFull) {
+      refill();
+      c = popc(__ballot(front != kEmptyKey));
+    }
+    return c;
+  }
+  // True if fewer than `limit` expanded keys lie below p, which is at or below
+  // every unexpanded key but those before it in `front`.
+  __device__ __forceinline__ bool fewer_below(uint64_t p, int limit) const {
+    int below = 0;
+    for (int c = 0; c < nbuf; c += 64) {
+      const int i = c + int(__lane_id());
+      below += popc(__ballot(i < nbuf && buf[i < nbuf ? i : 0] < p));
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) below += popc(__ballot(rest[e] < p));
+    return below < limit;
+  }
+  // The first `count` entries of `front` are expanded.
+  __device__ __forceinline__ void expand(int count) {
+    const int lane = __lane_id();
+    if (lane < count) buf[nbuf + lane] = front | 1ull;
+    nbuf += count;
+    expanded += count;
+    const uint64_t up = shfl_u64(front, (lane + count) & 63);
+    front = lane + count < 64 ? up : kEmptyKey;
+  }
+  // Keys on their way into `rest`, one per lane (the empty key for none).
+  __device__ __forceinline__ void push(uint64_t key) {
+    const uint64_t m = __ballot(key != kEmptyKey);
+    if (m == 0) return;
+    if (key != kEmptyKey) buf[nbuf + mbcnt(m)] = key;
+    nbuf += popc(m);
+    const uint32_t hi = wave_min_u32(uint32_t(key >> 32));
+    const uint32_t lo = wave_min_u32(uint32_t(key >> 32) == hi ? uint32_t(key) : 0xffffffffu);
+    const uint64_t low = (uint64_t(hi) << 32) | lo;
+    flim = low < flim ? low : flim;
+  }
+  // Candidate keys, one per lane (the empty key for none).
+  __device__ __forceinline__ void add(uint64_t key) {
+    push(key < flim ? kEmptyKey : key);
+    if (sort_below(key, flim, kEmptyKey, buf + kBuf) == 0) return;
+    // The 64 smallest of both stay; min and max of one ascending and one
+    // descending list are its halves, the lower one bitonic.
+    const int lane = __lane_id();
+    const uint64_t other = shfl_xor_u64(key, 63);  // lane 63 - lane
+    const uint64_t up = front < other ? other : front;
+    front = front < other ? front : other;
+#pragma unroll
+    for (int stride = 32; stride >= 1; stride >>= 1) {
+      const uint64_t y = shfl_xor_u64(front, stride);
+      front = ((lane & stride) == 0) == (front < y) ? front : y;
+    }
+    push(up);
+  }
+};
+
+// The same search for batches that leave compute units idle (W = 4 or 8,
+// d <= 1024, bitmap visited set, degree <= 64, width <= kAhead, one team),
+// where one query's chain of dependent steps is the time: per expanded node
+// the graph row, the visited test, the rows, the merge (3.1 us a node at
+// N=100K D=1024 fp32, of which the row bytes take 0.45 us at one compute
+// unit's load bandwidth).  Here one step serves several nodes:
+//  - the lead wave takes the `ahead` nearest unexpanded entries;
+//  - the neighbours of those whose neighbours are not at hand yet are
+//    collected (one entry per wave) and their rows gathered together, and
+//    their keys kept per entry in one of kAhead slots;
+//  - as many of the entries are expanded as the search would have expanded
+//    one iteration after the other: iteration i + 1 takes the next `width`
+//    entries iff no candidate of the iterations before is nearer than the
+//    last of them.  Their candidates join the visited set and the pool
+//    together; the other entries go back, their keys stay in their slots.
+// An entry near the head of the list is nearly always expanded soon, so few
+// evaluations are lost.  Parents, visited set, list and counts are, iteration
+// by iteration, those of cagra_search_kernel.
+// A call at N=100K D=1024 fp32: itopk 64 Q=1 213 -> 185 us in 20 steps for 65
+// nodes, itopk 512 Q=100 1611 -> 806 us in 81 steps for 512.  Of the latter's
+// 21,600 cycles a step, 7,700 are the gathers (27 rows; the latency of one
+// alone is 4,700), 4,500 the entries' choice and the pool's refills, 2,300
+// the new candidates, 2,400 the run of iterations and the visited set, 1,900
+// the graph rows: latencies of single instructions of one wave for the most
+// part.
+constexpr int kAhead = 8;         // entries with keys at hand
+constexpr int kAheadHash = 1024;  // ids of one step: at most kAhead * 64, half full
+
+template <int E, int W, bool F16>
+__global__ __launch_bounds__(64 * W, 2) void cagra_ahead_kernel(SearchArgs a, int ahead) {
+  extern __shared__ uint32_t s_mem[];
+  constexpr int kThreads = 64 * W, kTeams = 4 * W;
+  constexpr int kIds = kAhead * 64;      // candidates of one step
+  constexpr int kPerWave = kAhead / W;   // entries per wave and step
+  static_assert(kPerWave * W == kAhead, "entries per wave");
+  uint32_t* s_bits = s_mem;                               // visited rows (bitmap_words: whole 256-byte blocks)
+  uint64_t* s_key = reinterpret_cast<uint64_t*>(s_bits + a.bitmap_words);  // [slot][64] keys
+  uint32_t* s_ids = reinterpret_cast<uint32_t*>(s_key + kIds);
+  float* s_dist = reinterpret_cast<float*>(s_ids + kIds);
+  uint32_t* s_hid = reinterpret_cast<uint32_t*>(s_dist + kIds);  // ids of this step -> position in s_ids
+  uint32_t* s_hpos = s_hid + kAheadHash;
+  uint64_t* s_cand = reinterpret_cast<uint64_t*>(s_ids);  // candidates of a step's expanded entries (ids and distances are done with)
+  uint64_t* s_pick = reinterpret_cast<uint64_t*>(s_hpos + kAheadHash);  // keys of this step's entries
+  uint32_t* s_slot = reinterpret_cast<uint32_t*>(s_pick + kAhead);      // their slots
+  uint32_t* s_min = s_slot + kAhead;  // smallest distance word among an entry's unvisited neighbours
+  // [0] entries of this step, [1] mask of those to collect for, [2] how many of
+  // the first `width` are in the list, [3] most entries to expand, [4, 5] the
+  // pool's bound, [6] seeds, then candidates, [7] ids of this step, [8]
+  // distance evaluations
+  uint32_t* s_ctl = s_min + kAhead;
+  uint64_t* s_pool = reinterpret_cast<uint64_t*>(s_ctl + 16);
+  float* s_q = reinterpret_cast<float*>(s_pool + Pool<E>::kLds + 1);  // fp16 traversal: the query, kBigDim floats
+  const int tid = threadIdx.x, lane = tid & 63, team = tid >> 4, tp = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool lead = wave == 0;
+  const int64_t qi = blockIdx.x / a.teams;
+  const int tm = int(blockIdx.x - qi * a.teams);
+  const float* qsrc = a.queries + qi * a.d;
+
+  for (int i = tid; i < a.bitmap_words; i += kThreads) s_bits[i] = 0u;
+  for (int i = tid; i < kAheadHash; i += kThreads) s_hid[i] = kInvalidId;
+  if (tid < 16) s_ctl[tid] = 0u;
+  Slice<F16> slice;
+  slice.load(a, qsrc, tp);
+  if constexpr (F16) stage_query(a, qsrc, s_q, kThreads);
+
+  // Distances of the rows s_ids[0..nf) into s_dist, two rows in flight per team.
+  auto evaluate = [&](int nf) {
+    using Piece = typename Slice<F16>::Piece;
+    int r0 = 0;
+    for (; nf - r0 > kTeams; r0 += 2 * kTeams) {
+      const int ra = r0 + team, rb = ra + kTeams;
+      Piece xa[Slice<F16>::N], xb[Slice<F16>::N];
+      slice.fetch(a, s_ids[ra], tp, xa);
+      slice.fetch(a, s_ids[rb < nf ? rb : ra], tp, xb);
+      const float da = team_sum(slice.part(a, xa)), db = team_sum(slice.part(a, xb));
+      if (tp == 0) {
+        s_dist[ra] = da;
+        if (rb < nf) s_dist[rb] = db;
+      }
+    }
+    if (r0 < nf) {
+      const int r = r0 + team;
+      Piece x[Slice<F16>::N];
+      slice.fetch(a, s_ids[r < nf ? r : r0], tp, x);
+      const float d = team_sum(slice.part(a, x));
+      if (tp == 0 && r < nf) s_dist[r] = d;
+    }
+  };
+  auto visit = [&](uint32_t id) -> bool {  // true if id was not visited
+    const uint32_t bit = 1u << (id & 31u);
+    return (atomicOr(&s_bits[id >> 5], bit) & bit) == 0u;
+  };
+
+  Pool<E> pool;  // the list (lead wave)
+  pool.init(a.itopk, s_pool);
+  uint32_t sp = kInvalidId;  // lead wave, lane l < kAhead: the entry whose neighbours' keys slot l holds
+
+  // Seeds (the sequence of cagra_search_kernel), kIds at a time.
+  const uint32_t h0 = uint32_t(qi) * 2654435761u;
+  uint32_t* s_raw = reinterpret_cast<uint32_t*>(s_dist);
+  for (int c0 = 0; c0 < a.seed_lanes; c0 += kIds) {
+    const int cnt = a.seed_lanes - c0 < kIds ? a.seed_lanes - c0 : kIds;
+    for (int i = tid; i < cnt; i += kThreads) {
+      const int x = (c0 + i) * a.teams + tm;
+      uint32_t id = kInvalidId;
+      if (x < a.n_seeds)
+        id = a.seeds[x];
+      else if (uint32_t(x - a.n_seeds) < a.n)
+        id = (h0 + uint32_t(x - a.n_seeds) * 0x9E3779B9u) % a.n;
+      s_raw[i] = id;
+    }
+    __syncthreads();
+    if (lead) {
+      int nf = 0;
+      for (int c = 0; c < cnt; c += 64) {  // cnt is a multiple of 64
+        const uint32_t id = s_raw[c + lane];
+        const bool fresh = id < a.n && visit(id);
+        const uint64_t m = __ballot(fresh);
+        if (fresh) s_ids[nf + mbcnt(m)] = id;
+        nf += popc(m);
+      }
+      if (lane == 0) {
+        s_ctl[6] = uint32_t(nf);
+        s_ctl[8] += uint32_t(nf);
+      }
+    }
+    __syncthreads();
+    const int nf = int(s_ctl[6]);
+    evaluate(nf);
+    __syncthreads();
+    // Each wave sorts its 64-key runs, the lead wave merges them.
+    for (int b = wave * 64; b < nf; b += W * 64) {
+      const int i = b + lane;
+      s_key[i] = wave_sort_lanes<64>(
+          i < nf ? (uint64_t(ord_f32(s_dist[i])) << 32) | (uint64_t(s_ids[i]) << 1) : kEmptyKey);
+    }
+    __syncthreads();
+    if (lead)
+      for (int b = 0; b < nf; b += 64) pool.merge_sorted(s_key[b + lane]);
+    __syncthreads();  // the next seeds are staged over the distances
   }
 
-  if (lead && a.team_keys) {
+  int it = 0;
+  for (;;) {
+    if (lead) {
+      int n = 0, first = 0, most = 0;
+      uint32_t miss = 0;
+      if (it < a.max_iter) {
+        n = min(pool.ready(ahead), ahead);
+        // Of the first `width` entries, those are parents that are in the
+        // list: with fewer than itopk expanded keys below, counting the
+        // parents before.  Later iterations are taken only where that is
+        // certain.
+        const int w = n < a.width ? n : a.width;
+        const int sure = a.itopk - pool.expanded;
+        for (; first < w; ++first)
+          if (first >= sure && !pool.fewer_below(shfl_u64(pool.front, first), a.itopk - first)) break;
+        most = first < a.width ? first : max(first, min(sure, n));
+        if (first == 0) n = 0;
+        // Lane i finds the slot that holds entry i's keys; entries without
+        // one get, in order, the slots that no entry of this step holds.
+        const uint32_t id = lane < n ? uint32_t(pool.front) >> 1 : kInvalidId - 1;
+        uint32_t slot = kAhead, keep = 0;
 #pragma unroll
-    for (int e = 0; e < E; ++e) {
-      const int pos = e * 64 + lane;
-      if (pos < a.itopk) a.team_keys[int64_t(blockIdx.x) * a.itopk + pos] = top[e];
-    }
-  } else if (lead) {
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-      const int pos = e * 64 + lane;
-      if (pos < a.k) {
-        const uint64_t key = top[e];
-        a.out_nbr[qi * a.k + pos] = key == kEmptyKey ? kInvalidId : uint32_t(key) >> 1;
-        a.out_dist[qi * a.k + pos] = key == kEmptyKey ? INFINITY : unord_f32(uint32_t(key >> 32));
+        for (int l = 0; l < kAhead; ++l) {
+          const bool mine = id == uint32_t(__builtin_amdgcn_readlane(int(sp), l));
+          slot = mine ? uint32_t(l) : slot;
+          keep |= __ballot(mine) != 0 ? 1u << l : 0u;
+        }
+        miss = uint32_t(__ballot(lane < n && slot == uint32_t(kAhead)));
+        if (miss != 0) {
+          const bool free = lane < kAhead && ((keep >> (lane & 31)) & 1u) == 0u;
+          const int nth = mbcnt(__ballot(free));  // slot `lane` is the nth free one,
+          if (free) s_slot[nth] = uint32_t(lane);
+          if (slot == uint32_t(kAhead) && lane < n) {
+            slot = s_slot[mbcnt(uint64_t(miss))];
+            s_min[slot] = id;  // and takes the nth of these entries
+          }
+          if (free && nth < popc(uint64_t(miss))) sp = s_min[lane];
+        }
+        if (lane < n) {
+          s_pick[lane] = pool.front;
+          s_slot[lane] = slot;
+        }
+      }
+      if (lane == 0) {
+        *reinterpret_cast<uint4*>(s_ctl) = uint4{uint32_t(n), miss, uint32_t(first), uint32_t(most)};
+        *reinterpret_cast<uint4*>(s_ctl + 4) = uint4{uint32_t(pool.bound), uint32_t(pool.bound >> 32), 0u, 0u};
       }
     }
-    if (a.stats && lane == 0) {
-      a.stats[2 * qi] = evals;
-      a.stats[2 * qi + 1] = uint32_t(it);
+    __syncthreads();
+    const uint4 ctl = *reinterpret_cast<const uint4*>(s_ctl);
+    const int n = __builtin_amdgcn_readfirstlane(int(ctl.x));
+    const uint32_t miss = uint32_t(__builtin_amdgcn_readfirstlane(int(ctl.y)));
+    if (n == 0) break;
+    // Each wave serves its entries of the step: the keys of their neighbours
+    // from their slots, or collected and gathered.
+    uint64_t key[kPerWave];
+    uint32_t id[kPerWave], slot[kPerWave];
+    int pos[kPerWave];  // collected: hash position, -1: no candidate
+#pragma unroll
+    for (int t = 0; t < kPerWave; ++t) {
+      const int p = wave + t * W;
+      key[t] = kEmptyKey;
+      id[t] = kInvalidId;
+      slot[t] = 0;
+      if (p < n) {
+        slot[t] = s_slot[p];
+        if ((miss >> p) & 1u) {
+          if (lane < a.g) id[t] = a.graph[int64_t(uint32_t(s_pick[p]) >> 1) * a.g + lane];
+        } else {
+          key[t] = s_key[slot[t] * 64 + lane];
+          id[t] = uint32_t(key[t]) >> 1;  // >= n for none
+        }
+      }
+    }
+    bool open[kPerWave];  // not visited
+#pragma unroll
+    for (int t = 0; t < kPerWave; ++t)
+      open[t] = id[t] < a.n && ((s_bits[id[t] < a.n ? id[t] >> 5 : 0] >> (id[t] & 31u)) & 1u) == 0u;
+    if (miss != 0) {
+      // Each id of the step once.
+#pragma unroll
+      for (int t = 0; t < kPerWave; ++t) {
+        pos[t] = -1;
+        if (((miss >> (wave + t * W)) & 1u) == 0) continue;
+        bool first_seen = false;
+        if (open[t]) {
+          uint32_t h = (id[t] * 0x9E3779B1u) >> 22;  // kAheadHash positions
+          for (;;) {
+            const uint32_t old = atomicCAS(&s_hid[h], kInvalidId, id[t]);
+            first_seen = old == kInvalidId;
+            if (first_seen || old == id[t]) break;
+            h = (h + 1u) & uint32_t(kAheadHash - 1);
+          }
+          pos[t] = int(h);
+        }
+        const uint64_t m = __ballot(first_seen);
+        if (m != 0) {
+          uint32_t base = 0;
+          if (lane == 0) base = atomicAdd(&s_ctl[7], uint32_t(popc(m)));
+          base = uint32_t(__builtin_amdgcn_readfirstlane(int(base)));
+          if (first_seen) {
+            const uint32_t at = base + uint32_t(mbcnt(m));
+            s_ids[at] = id[t];
+            s_hpos[pos[t]] = at;
+          }
+        }
+      }
+      __syncthreads();
+      evaluate(int(s_ctl[7]));
+      __syncthreads();
+#pragma unroll
+      for (int t = 0; t < kPerWave; ++t) {
+        if (((miss >> (wave + t * W)) & 1u) == 0) continue;
+        if (pos[t] >= 0) key[t] = (uint64_t(ord_f32(s_dist[s_hpos[pos[t]]])) << 32) | (uint64_t(id[t]) << 1);
+        s_key[slot[t] * 64 + lane] = key[t];
+      }
+    }
+    // The nearest unvisited neighbour of each entry.
+#pragma unroll
+    for (int t = 0; t < kPerWave; ++t) {
+      const int p = wave + t * W;
+      if (!open[t]) key[t] = kEmptyKey;
+      const uint32_t mn = wave_min_u32(uint32_t(key[t] >> 32));
+      if (lane == 0 && p < n) s_min[p] = mn;
+    }
+    __syncthreads();
+    // The iterations that follow one another whatever their candidates are
+    // (equal distances end the run; the next step then looks at the ids):
+    // entry j ends an iteration that may follow if the nearest neighbour of
+    // all iterations before it lies beyond it.
+    int c = __builtin_amdgcn_readfirstlane(int(ctl.z)), iters = 1;
+    {
+      const int most = __builtin_amdgcn_readfirstlane(int(ctl.w));
+      uint32_t before = lane < n ? s_min[lane & (kAhead - 1)] : 0xffffffffu;  // of entries 0 .. lane
+      const uint32_t own = uint32_t(s_pick[lane & (kAhead - 1)] >> 32);
+      // Running minimum by DPP row shifts (kAhead lanes of the first row).
+      static_assert(kAhead == 8, "three row shifts");
+      before = min(before, uint32_t(__builtin_amdgcn_update_dpp(-1, int(before), 0x111, 0xF, 0xF, false)));
+      before = min(before, uint32_t(__builtin_amdgcn_update_dpp(-1, int(before), 0x112, 0xF, 0xF, false)));
+      before = min(before, uint32_t(__builtin_amdgcn_update_dpp(-1, int(before), 0x114, 0xF, 0xF, false)));
+      before = a.width == 1 ? uint32_t(__builtin_amdgcn_update_dpp(-1, int(before), 0x111, 0xF, 0xF, false))
+                            : uint32_t(__shfl_up(int(before), a.width));
+      const uint64_t ok = __ballot(lane >= a.width && lane < most && before > own);
+      while (c + a.width <= most && it + iters < a.max_iter && ((ok >> (c + a.width - 1)) & 1ull)) {
+        c += a.width;
+        ++iters;
+      }
+    }
+    it += iters;
+    if (miss != 0)  // empty for the next step, which starts with a barrier
+      for (int i = tid; i < kAheadHash; i += kThreads) s_hid[i] = kInvalidId;
+    const uint64_t bound = *reinterpret_cast<const uint64_t*>(s_ctl + 4);
+#pragma unroll
+    for (int t = 0; t < kPerWave; ++t) {
+      if (wave + t * W >= c) continue;
+      const bool fresh = key[t] != kEmptyKey && visit(id[t]);
+      const uint64_t m = __ballot(fresh && key[t] < bound);
+      const int nfresh = popc(__ballot(fresh));
+      uint32_t base = 0;
+      if (lane == 0) {
+        base = atomicAdd(&s_ctl[6], uint32_t(popc(m)));
+        atomicAdd(&s_ctl[8], uint32_t(nfresh));
+      }
+      base = uint32_t(__builtin_amdgcn_readfirstlane(int(base)));
+      if ((m >> lane) & 1ull) s_cand[base + mbcnt(m)] = key[t];
+    }
+    __syncthreads();
+    if (lead) {
+      const int nc = int(s_ctl[6]);
+      // The expanded entries' slots are free.
+      for (int i = 0; i < c; ++i) {
+        const uint32_t x = uint32_t(__builtin_amdgcn_readlane(int(uint32_t(pool.front)), i)) >> 1;
+        sp = sp == x ? kInvalidId : sp;
+      }
+      pool.expand(c);
+      for (int b = 0; b < nc; b += 64) pool.add(b + lane < nc ? s_cand[b + lane] : kEmptyKey);
     }
   }
+
+  if (lead) pool.collect();
+  if constexpr (F16)
+    rerank_list<E, W>(pool.rest, lead, s_ids, s_dist,
+                      [&](uint32_t rid) { return team_sum(exact_part(a, s_q, rid, tp)); });
+  if (lead) write_list<E>(a, pool.rest, qi, s_ctl[8], it);
 }
 
 // Waves per query (workgroups = queries x teams): 8 up to 128 workgroups, 4
@@ -561,8 +1186,18 @@ int waves_per_query(int64_t workgroups) {
 }
 
 template <int E, bool F16>
-void launch_search(int waves, bool big, dim3 grid, size_t lds, hipStream_t stream, const SearchArgs& a,
+void launch_search(int waves, bool big, int ahead, dim3 grid, size_t lds, hipStream_t stream, const SearchArgs& a,
                    hipEvent_t e0, hipEvent_t e1) {
+  if (ahead > 0 && waves == 8) {
+    hipExtLaunchKernelGGL((cagra_ahead_kernel<E, 8, F16>), grid, dim3(512), lds, stream, e0, e1, 0, a, ahead);
+    return;
+  }
+  if constexpr (E > 1) {
+    if (ahead > 0) {
+      hipExtLaunchKernelGGL((cagra_ahead_kernel<E, 4, F16>), grid, dim3(256), lds, stream, e0, e1, 0, a, ahead);
+      return;
+    }
+  }
   if (big) {  // d > 1024: four waves per query at any batch size
     if (lds > 64 * 1024)
       CVS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(cagra_search_kernel<E, 4, F16, true>),
@@ -578,12 +1213,12 @@ void launch_search(int waves, bool big, dim3 grid, size_t lds, hipStream_t strea
 }
 
 template <int E>
-void launch_search(bool f16, int waves, bool big, dim3 grid, size_t lds, hipStream_t stream, const SearchArgs& a,
-                   hipEvent_t e0, hipEvent_t e1) {
+void launch_search(bool f16, int waves, bool big, int ahead, dim3 grid, size_t lds, hipStream_t stream,
+                   const SearchArgs& a, hipEvent_t e0, hipEvent_t e1) {
   if (f16)
-    launch_search<E, true>(waves, big, grid, lds, stream, a, e0, e1);
+    launch_search<E, true>(waves, big, ahead, grid, lds, stream, a, e0, e1);
   else
-    launch_search<E, false>(waves, big, grid, lds, stream, a, e0, e1);
+    launch_search<E, false>(waves, big, ahead, grid, lds, stream, a, e0, e1);
 }
 
 // Merge of the teams' lists of one query (one wave per query): the teams x
@@ -788,9 +1423,28 @@ void cagra_search_device(cvs_context* ctx, const cvs_cagra_index* idx, const flo
   const int64_t bitmap_words = (idx->n + 2047) / 2048 * 64;
   const bool use_bitmap = bitmap_words <= (int64_t(1) << hash_bits);
   const size_t visit_words = use_bitmap ? size_t(bitmap_words) : (size_t(1) << hash_bits);
-  const size_t lds = visit_words * 4 + (64 + 64 + CVS_CAGRA_MAX_WIDTH + 8) * 4 +
-                     (big ? size_t(idx->dpad) * 4 * (idx->traversal_bits == 16 ? 2 : 1)
-                          : (idx->traversal_bits == 16 ? size_t(kBigDim) * 4 : 0));
+  // Small batches gather for several entries at a time (cagra_ahead_kernel)
+  // where that is the faster way.  It pays once the list is long enough that
+  // most expansions are of entries already in it: at N=100K D=1024 fp32,
+  // without and with it, itopk 32 Q=1 125 / 147 us (not taken), 64 Q=1 213 /
+  // 185, Q=128 265 / 246, 128 Q=1 414 / 244, 512 Q=100 1611 / 806.  With four
+  // waves (129 to 512 queries) compute units are shared, and the rows that
+  // are gathered in vain cost more: itopk 64 Q=300 307 / 359 (not taken), 128
+  // Q=200 500 / 435, Q=500 545 / 534, 512 Q=500 1534 / 1077.  Teams walk from
+  // scattered seeds with short lists (8 teams x 32, Q=1: 123 / 175; 4 x 64:
+  // 213 / 250; not taken), and beyond 512 workgroups it is slower at any
+  // itopk (512 Q=1,000: 1737 / 2038).  Six entries are best for one key per
+  // lane (4: 196, 8: 192 us at Q=1), eight for longer lists.
+  int ahead = 0;
+  if (waves >= 4 && !big && use_bitmap && idx->degree <= 64 && width <= kAhead && teams == 1 && !record &&
+      itopk > (waves == 8 ? 32 : 64))
+    ahead = std::max(itopk > 64 ? kAhead : 6, int(width));
+  const bool f16 = idx->traversal_bits == 16;
+  size_t lds = visit_words * 4 + (64 + 64 + CVS_CAGRA_MAX_WIDTH + 8) * 4 +
+               (big ? size_t(idx->dpad) * 4 * (f16 ? 2 : 1) : (f16 ? size_t(kBigDim) * 4 : 0));
+  if (ahead > 0)  // the kernel's arrays, in its order
+    lds = visit_words * 4 + size_t(kAhead * 64) * 16 + size_t(kAheadHash) * 8 + (4 * kAhead + 16) * 4 +
+          size_t(Pool<1>::kLds + 64 * (e_slots - 1) + 1) * 8 + (f16 ? size_t(kBigDim) * 4 : 0);
 
   SearchArgs a{};
   a.rows = reinterpret_cast<const float4*>(idx->rows);
@@ -833,14 +1487,13 @@ void cagra_search_device(cvs_context* ctx, const cvs_cagra_index* idx, const flo
 
   const TimerSpan t0 = timer_span(ctx, "cagra_search");
   const dim3 grid(static_cast<unsigned>(q * teams));
-  const bool f16 = idx->traversal_bits == 16;
   // The search kernel starts the span; the team merge (if any) ends it.
   hipEvent_t e1 = teams > 1 ? nullptr : t0.stop;
   switch (e_slots) {
-    case 1: launch_search<1>(f16, waves, big, grid, lds, ctx->stream, a, t0.start, e1); break;
-    case 2: launch_search<2>(f16, waves, big, grid, lds, ctx->stream, a, t0.start, e1); break;
-    case 4: launch_search<4>(f16, waves, big, grid, lds, ctx->stream, a, t0.start, e1); break;
-    default: launch_search<8>(f16, waves, big, grid, lds, ctx->stream, a, t0.start, e1); break;
+    case 1: launch_search<1>(f16, waves, big, ahead, grid, lds, ctx->stream, a, t0.start, e1); break;
+    case 2: launch_search<2>(f16, waves, big, ahead, grid, lds, ctx->stream, a, t0.start, e1); break;
+    case 4: launch_search<4>(f16, waves, big, ahead, grid, lds, ctx->stream, a, t0.start, e1); break;
+    default: launch_search<8>(f16, waves, big, ahead, grid, lds, ctx->stream, a, t0.start, e1); break;
   }
   after_launch("cagra_search_kernel");
   if (teams > 1) {
