@@ -69,18 +69,23 @@ using namespace bf;
 constexpr int kThreads = 256;  // 4 waves
 constexpr int kWaves = 4;
 constexpr int kQB = 128;                                // queries per workgroup (32 per wave)
-constexpr int kStageBlocks = 32;                        // 1 KiB blocks per stage
-constexpr int kStageVecs = kStageBlocks * 64;           // 16-byte vectors per stage
-constexpr int kLoadsPerThread = kStageVecs / kThreads;  // 8 16-byte loads per thread and stage
 
+// Stages of the scan over tiles of KS k-steps: SB 1 KiB blocks, a tile (KS 20
+// to 32), half a tile (beyond) or as many tiles as 32 blocks hold.  SB is a
+// multiple of 4 (whole loads of 256 threads) and at least 20 (the pipelined
+// loop's slots), which is what sets the padded dimensions (padded_dim).
 template <int KS>
 struct Cfg {
-  static constexpr int TPS = KS >= 32 ? 1 : 32 / KS;      // tiles per stage
-  static constexpr int SPT = KS >= 32 ? KS / 32 : 1;      // stages per tile
-  static constexpr int RPU = 2 * kStageBlocks * 32 / KS;  // rows per 2-stage unit
-  static constexpr int NF = TPS * 32;                     // norms per stage
-  static_assert(KS >= 2 && KS <= 64, "k-steps per tile");
+  static constexpr int TPS = KS >= 20 ? 1 : 32 / KS;  // tiles per stage
+  static constexpr int SPT = KS > 32 ? 2 : 1;         // stages per tile
+  static constexpr int SB = KS * TPS / SPT;           // 1 KiB blocks per stage
+  static constexpr int VECS = SB * 64;                // 16-byte vectors per stage
+  static constexpr int LPT = VECS / kThreads;         // 16-byte loads per thread and stage
+  static constexpr int NF = TPS * 32;                 // norms per stage
+  static_assert(KS >= 2 && KS <= 64 && SB % 4 == 0 && SB >= 20 && SB <= 32, "k-steps per tile");
 };
+// Tiles of a two-stage unit (the scan's unit of work), the same on the host.
+constexpr int tiles_per_unit(int ks) { return ks > 32 ? 1 : (ks >= 20 ? 2 : 2 * (32 / ks)); }
 
 struct ScanArgs {
   const u32x4* tiles;   // dataset tiles (unit-padded)
@@ -111,9 +116,10 @@ void bf_scan_kernel(ScanArgs a) {
   using C = Cfg<KS>;
   using L = Lists<KP, MODE>;
   constexpr int TPS = C::TPS, SPT = C::SPT, NF = C::NF;
+  constexpr int kStageBlocks = C::SB, kStageVecs = C::VECS, kLoadsPerThread = C::LPT;
   constexpr int CAP = L::CAP;
-  // Scans over 32 or 64 k-steps per tile run the software-pipelined loop.
-  constexpr bool PIPE = MODE == kModeScan && KS >= 32;
+  // Scans over 20 or more k-steps per tile run the software-pipelined loop.
+  constexpr bool PIPE = MODE == kModeScan && KS >= 20;
 
   __shared__ u32x4 s_stage[2][kStageVecs];
   __shared__ float s_dn[2][NF];
@@ -154,7 +160,7 @@ void bf_scan_kernel(ScanArgs a) {
     const u32x4* src = a.tiles + st * kStageVecs + tid;
 #pragma unroll
     for (int i = 0; i < kLoadsPerThread; ++i) r[i] = __builtin_nontemporal_load(src + i * kThreads);
-    const int64_t tile0 = KS >= 32 ? st / SPT : st * TPS;
+    const int64_t tile0 = KS >= 20 ? st / SPT : st * TPS;
     const float* ns = reinterpret_cast<const float*>(a.norms) + tile0 * 32;
 #pragma unroll
     for (int i = 0; i < NPT; ++i)
@@ -353,8 +359,8 @@ void bf_scan_kernel(ScanArgs a) {
     const u32x4* sb = s_stage[buf] + lane;
     const float* dn = s_dn[buf];
     (void)st;
-    if constexpr (KS >= 32) {
-      // One stage is 32 k-steps of a single tile.
+    if constexpr (KS >= 20) {
+      // One stage is a tile or half of one.
       constexpr int KOFF = (PAR * kStageBlocks) % KS;
       mfma_run(sb, std::integral_constant<int, kStageBlocks>{}, std::integral_constant<int, KOFF>{});
       if constexpr (KOFF + kStageBlocks == KS) epilogue(dn, (st / SPT) * 32, j);
@@ -385,10 +391,10 @@ void bf_scan_kernel(ScanArgs a) {
       step(std::integral_constant<int, 1>{}, rb, nb, j + 1);
     }
   } else {
-    // ---- software-pipelined scan (32 or 64 k-steps per tile) ----
+    // ---- software-pipelined scan (20 or more k-steps per tile) ----
     // Stage j sits in LDS buffer j&1 and, until it is stored there, in
     // register set j&1 (ra / rb).  Per stage, after one barrier, a single scheduling region
-    // interleaves with the stage's 32 MFMAs: the previous tile's
+    // interleaves with the stage's SB MFMAs: the previous tile's
     // distance/threshold test (VALU), the LDS store of stage j+1 (its buffer
     // was last read in stage j-1, which every wave finished before the
     // barrier) and the HBM load of stage j+3 into the registers just stored.
@@ -426,14 +432,20 @@ void bf_scan_kernel(ScanArgs a) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) dv[r] = 0.f;
 
-    // One stage as 32 slots separated by scheduling fences, so that the
+    // One stage as SB slots separated by scheduling fences, so that the
     // interleave is fixed: slot i issues MFMA i, the LDS read of block i+8
     // (8-deep A ring, two accumulation chains), and one piece of the side
     // work.  Slot 0 of a tile's first stage first sums the previous tile's
-    // two chains and slots 8-11 read that tile's norms from LDS; slots 12-19
-    // store stage j+1 to LDS and reuse each register for stage j+3; slot 20
-    // stores a tile's norms, slot 21 loads them; slots 16-31 of a first stage
-    // turn the previous tile's dot products into distances and pass bits.
+    // two chains and four slots read that tile's norms from LDS (8-11 of 32);
+    // the next (12-19 of 32) store stage j+1 to LDS and reuse each register
+    // for stage j+3; one stores a tile's norms (20), one loads them (21); the
+    // last 16 of a first stage turn the previous tile's dot products into
+    // distances and pass bits.  Stages of 28, 24 and 20 blocks shift all of
+    // it forward by as many slots as they are shorter (the norms' reads no
+    // further than slot 0).
+    constexpr int kCut = 32 - kStageBlocks;
+    constexpr int kNormRead = kCut > 8 ? 0 : 8 - kCut, kSwap = 12 - kCut, kNormStore = 20 - kCut,
+                  kDist = 16 - kCut;
     auto pstep = [&](auto par_c, u32x4 (&r)[kLoadsPerThread], float& rn, int j) CVS_INLINE {
       constexpr int PAR = decltype(par_c)::value;
       constexpr bool FIRST = SPT == 1 || PAR == 0;    // first stage of its tile
@@ -466,27 +478,27 @@ void bf_scan_kernel(ScanArgs a) {
         else
           acc0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, qb[KOFF + i], (FIRST && i < 2) ? zero : acc0, 0, 0, 0);
         if constexpr (FIRST) {
-          if (i >= 8 && i < 12) {
-            const int g = i - 8;
+          if (i >= kNormRead && i < kNormRead + 4) {
+            const int g = i - kNormRead;
             // Slot of tile tl-1 (for the first tile: never written, masked below).
             dn4[g] = *reinterpret_cast<const f32x4*>(dn_slot(tl + 3) + 8 * g + 4 * (lane >> 5));
           }
         }
-        if (i >= 12 && i < 12 + kLoadsPerThread) {
-          const int e = i - 12;
+        if (i >= kSwap && i < kSwap + kLoadsPerThread) {
+          const int e = i - kSwap;
           s_stage[PAR ^ 1][tid + e * kThreads] = r[e];  // past the last stage: zeros, never read
           r[e] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
                                                rsrc, off + uint32_t(e * kThreads * 16), 0, kAuxNT));
         }
         if constexpr (STORE_N) {
-          if (i == 20) dn_slot((j + 1) / SPT)[lane & 31] = rn;
+          if (i == kNormStore) dn_slot((j + 1) / SPT)[lane & 31] = rn;
         }
         if constexpr (LOAD_N) {
-          if (i == 21) rn = nload(j + 3);
+          if (i == kNormStore + 1) rn = nload(j + 3);
         }
         if constexpr (FIRST) {
-          if (i >= 16) {
-            const int q = i - 16;
+          if (i >= kDist) {
+            const int q = i - kDist;
             dv[q] = qn + dn4[q >> 2][q & 3] - 2.0f * dv[q];
             pass |= (dv[q] < thr ? 1u : 0u) << q;
           }
@@ -1178,27 +1190,20 @@ int choose_kp(int64_t k) {
   return 128;
 }
 
-template <int KS, int KP>
-void launch_scan_kp(cvs_context* ctx, dim3 grid, const ScanArgs& args, int mode, hipEvent_t e0, hipEvent_t e1) {
-  if (mode == kModeScan)
-    hipExtLaunchKernelGGL((bf_scan_kernel<KS, kModeScan, KP>), grid, dim3(kThreads), 0, ctx->stream, e0, e1, 0,
-                          args);
-  else
-    hipExtLaunchKernelGGL((bf_scan_kernel<KS, kModeSample, KP>), grid, dim3(kThreads), 0, ctx->stream, e0, e1, 0,
-                          args);
-}
-
 template <int KS>
 void launch_scan_ks(cvs_context* ctx, dim3 grid, const ScanArgs& args, int mode, hipEvent_t e0, hipEvent_t e1) {
+  auto launch = [&](auto kernel) {
+    hipExtLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, ctx->stream, e0, e1, 0, args);
+  };
   if (mode == kModeSample) {
-    launch_scan_kp<KS, 16>(ctx, grid, args, mode, e0, e1);  // list geometry unused when sampling
+    launch(bf_scan_kernel<KS, kModeSample, 16>);  // list geometry unused when sampling
     return;
   }
   switch (args.kp) {
-    case 16: launch_scan_kp<KS, 16>(ctx, grid, args, mode, e0, e1); break;
-    case 32: launch_scan_kp<KS, 32>(ctx, grid, args, mode, e0, e1); break;
-    case 64: launch_scan_kp<KS, 64>(ctx, grid, args, mode, e0, e1); break;
-    case 128: launch_scan_kp<KS, 128>(ctx, grid, args, mode, e0, e1); break;
+    case 16: launch(bf_scan_kernel<KS, kModeScan, 16>); break;
+    case 32: launch(bf_scan_kernel<KS, kModeScan, 32>); break;
+    case 64: launch(bf_scan_kernel<KS, kModeScan, 64>); break;
+    case 128: launch(bf_scan_kernel<KS, kModeScan, 128>); break;
     default: fail(CVS_ERR_RUNTIME, "unsupported candidate count");
   }
 }
@@ -1211,8 +1216,15 @@ void launch_scan(cvs_context* ctx, int ks, dim3 grid, const ScanArgs& args, int 
     case 2: launch_scan_ks<2>(ctx, grid, args, mode, e0, e1); break;
     case 4: launch_scan_ks<4>(ctx, grid, args, mode, e0, e1); break;
     case 8: launch_scan_ks<8>(ctx, grid, args, mode, e0, e1); break;
+    case 12: launch_scan_ks<12>(ctx, grid, args, mode, e0, e1); break;
     case 16: launch_scan_ks<16>(ctx, grid, args, mode, e0, e1); break;
+    case 20: launch_scan_ks<20>(ctx, grid, args, mode, e0, e1); break;
+    case 24: launch_scan_ks<24>(ctx, grid, args, mode, e0, e1); break;
+    case 28: launch_scan_ks<28>(ctx, grid, args, mode, e0, e1); break;
     case 32: launch_scan_ks<32>(ctx, grid, args, mode, e0, e1); break;
+    case 40: launch_scan_ks<40>(ctx, grid, args, mode, e0, e1); break;
+    case 48: launch_scan_ks<48>(ctx, grid, args, mode, e0, e1); break;
+    case 56: launch_scan_ks<56>(ctx, grid, args, mode, e0, e1); break;
     case 64: launch_scan_ks<64>(ctx, grid, args, mode, e0, e1); break;
     default: fail(CVS_ERR_UNSUPPORTED, "unsupported padded dimension");
   }
@@ -1262,8 +1274,8 @@ BfPlan plan_bf(cvs_context* ctx, const cvs_dataset* ds, const float* queries, in
 
   BfPlan p;
   p.ks = int(ds->dp / kStepCols);
-  const int rpu = 2 * kStageBlocks * 32 / p.ks;  // rows per unit
-  p.n_units = ds->n_tiles * p.ks / (2 * kStageBlocks);
+  const int rpu = tiles_per_unit(p.ks) * int(kTileRows);  // rows per unit
+  p.n_units = ds->n_tiles / tiles_per_unit(p.ks);
   p.kp = choose_kp(k);
   p.qblocks = unsigned((q + kQB - 1) / kQB);
   const bool global_lists = p.kp > 64;

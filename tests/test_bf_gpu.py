@@ -116,6 +116,27 @@ def test_random_shapes(ctx, oracle, n, d, q, k):
     check_against_oracle(ctx, oracle, base, qs, k)
 
 
+@pytest.mark.parametrize("d", [129, 192, 193, 320, 321, 384, 385, 448, 449, 640, 641, 768, 769, 896, 897])
+@pytest.mark.parametrize("n,q,k", [
+    (17000, 33, 10), (9001, 130, 24), (6002, 5, 48), (4003, 20, 100),  # one list geometry each
+    (4100, 1100, 60),                                                  # the register-blocked scan
+    (2000, 3, 120),                                                    # the keys-matrix path
+])
+def test_every_padded_dimension(ctx, d, n, q, k):
+    """First and last dimension of each k-step count that is no power of two:
+    whole-number rows, so that distances are exact and ids equal those of a
+    sort by (distance, id)."""
+    rng = np.random.default_rng(d * 7 + n)
+    base = rng.integers(-8, 9, (n, d)).astype(np.float32)
+    qs = rng.integers(-8, 9, (q, d)).astype(np.float32)
+    nbr, dist = ctx.dataset(base).bf_search(qs, k)
+    key = ((qs.astype(np.float64) ** 2).sum(1)[:, None] - 2.0 * (qs.astype(np.float64) @ base.T.astype(np.float64))
+           + (base.astype(np.float64) ** 2).sum(1)[None, :]).astype(np.int64) * n + np.arange(n)[None, :]
+    near = np.sort(np.partition(key, k - 1, axis=1)[:, :k], axis=1)
+    np.testing.assert_array_equal(nbr, near % n)
+    np.testing.assert_array_equal(dist, near // n)
+
+
 @pytest.mark.parametrize("n,d,q,k", [
     (30000, 64, 1500, 10),    # > 8 query blocks: range-major launch, LDS lists
     (30000, 64, 1500, 100),   # range-major launch, global-memory lists (8 k-steps or fewer)
@@ -126,8 +147,8 @@ def test_random_shapes(ctx, oracle, n, d, q, k):
     (20000, 512, 5000, 112),  # 10 query blocks: two per XCD for XCDs 0 and 1, largest k
     (12000, 1024, 1300, 10),  # range-major pipelined scan (64 k-steps), kp = 16 LDS lists
     (12000, 512, 1100, 40),   # range-major pipelined scan (32 k-steps), kp = 64 LDS lists
-    (7000, 384, 1100, 100),   # d 384 padded to 512: 128 zero columns in every tile
-    (5000, 640, 1030, 50),    # d 640 padded to 1024; the last 512-query block holds one 32-query tile
+    (7000, 384, 1100, 100),   # 24 k-steps
+    (5000, 640, 1030, 50),    # 40 k-steps; the last 512-query block holds one 32-query tile
     (9000, 768, 1200, 112),   # d 768 padded to 1024, largest k
     (3000, 896, 2100, 77),    # d 896 padded to 1024, 5 query blocks
 ])
