@@ -204,9 +204,11 @@ __device__ __forceinline__ void add_keys(uint64_t (&top)[E], uint64_t key, int i
 // rows are: a piece's distance is four packed differences and four
 // fp32-accumulating dot2s, and the slice takes 32 VGPRs instead of 64.  The
 // traversal's distances only steer the search; the list is re-ranked against
-// the fp32 query and rows at the end.  Query loads are unconditional (column
-// clamped, the value masked by an AND of its bits), so that all are in flight
-// together, and four columns wide where the query's rows are 16-byte aligned.
+// the fp32 query and rows at the end.  The query comes from LDS, where
+// stage_query put it with coalesced loads of any alignment (column clamped,
+// the value masked by an AND of its bits, so that no load sits under a
+// condition and all are in flight together): a lane's own loads of its 64
+// scattered columns took 8 us of a single query's search.
 __device__ __forceinline__ float masked(float x, bool in) {
   return __uint_as_float(__float_as_uint(x) & (in ? 0xffffffffu : 0u));
 }
@@ -217,22 +219,6 @@ __device__ __forceinline__ float sum_sq4(float x, float y, float z, float w) {
   return __builtin_fmaf(x, x, __fmul_rn(y, y)) + __builtin_fmaf(z, z, __fmul_rn(w, w));
 }
 
-// Columns c .. c + 3 of a query, zero past d.
-__device__ __forceinline__ float4 query_cols(const SearchArgs& a, const float* qsrc, bool vec, int64_t c) {
-  float4 v;
-  if (vec) {  // d is a multiple of 4: all four columns or none
-    v = *reinterpret_cast<const float4*>(qsrc + (c < a.d ? c : 0));
-    return make_float4(masked(v.x, c < a.d), masked(v.y, c < a.d), masked(v.z, c < a.d), masked(v.w, c < a.d));
-  }
-  const int64_t e = a.d - 1;
-  v = make_float4(qsrc[c < e ? c : e], qsrc[c + 1 < e ? c + 1 : e], qsrc[c + 2 < e ? c + 2 : e],
-                  qsrc[c + 3 < e ? c + 3 : e]);
-  return make_float4(masked(v.x, c < a.d), masked(v.y, c + 1 < a.d), masked(v.z, c + 2 < a.d), masked(v.w, c + 3 < a.d));
-}
-__device__ __forceinline__ bool wide_query(const SearchArgs& a, const float* qsrc) {
-  return (a.d & 3) == 0 && (reinterpret_cast<uintptr_t>(qsrc) & 15) == 0;
-}
-
 template <bool F16>
 struct Slice;
 
@@ -241,14 +227,9 @@ struct Slice<false> {
   using Piece = float4;
   static constexpr int N = kMaxDv;
   float4 q[N];
-  __device__ __forceinline__ void load(const SearchArgs& a, const float* qsrc, int tp) {
-    if (wide_query(a, qsrc)) {
+  __device__ __forceinline__ void load(const float* s_q, int tp) {
 #pragma unroll
-      for (int j = 0; j < N; ++j) q[j] = query_cols(a, qsrc, true, int64_t(tp + 16 * j) * 4);
-    } else {
-#pragma unroll
-      for (int j = 0; j < N; ++j) q[j] = query_cols(a, qsrc, false, int64_t(tp + 16 * j) * 4);
-    }
+    for (int j = 0; j < N; ++j) q[j] = reinterpret_cast<const float4*>(s_q)[tp + 16 * j];
   }
   __device__ __forceinline__ void fetch(const SearchArgs& a, uint32_t rid, int tp, float4 (&x)[N]) const {
     const float4* row = a.rows + int64_t(rid) * a.dq + tp;
@@ -274,24 +255,14 @@ struct Slice<true> {
   using Piece = uint4;
   static constexpr int N = kMaxDv8;
   half8_t q[N];
-  __device__ __forceinline__ void load(const SearchArgs& a, const float* qsrc, int tp) {
-    if (wide_query(a, qsrc))
-      load_cols(a, qsrc, tp, true);
-    else
-      load_cols(a, qsrc, tp, false);
-  }
-  // Centred and scaled as the traversal copy is (distances in the traversal
-  // are scale^2 times the squared distance), rounded to fp16.  mu holds zeros
-  // past d.
-  __device__ __forceinline__ void load_cols(const SearchArgs& a, const float* qsrc, int tp, bool vec) {
+  // From the centred, scaled query, rounded to fp16.
+  __device__ __forceinline__ void load(const float* s_q, int tp) {
 #pragma unroll
     for (int j = 0; j < N; ++j) {
-      const int64_t c = int64_t(tp + 16 * j) * 8;
-      const float4* mu = reinterpret_cast<const float4*>(a.mu + (j < a.dv8 ? c : 0));
-      const float4 x = query_cols(a, qsrc, vec, c), y = query_cols(a, qsrc, vec, c + 4), mx = mu[0], my = mu[1];
-      const float v[8] = {x.x - mx.x, x.y - mx.y, x.z - mx.z, x.w - mx.w, y.x - my.x, y.y - my.y, y.z - my.z, y.w - my.w};
-#pragma unroll
-      for (int t = 0; t < 8; ++t) q[j][t] = _Float16(masked(v[t] * a.scale, c + t < a.d));
+      const float4* v = reinterpret_cast<const float4*>(s_q + (tp + 16 * j) * 8);
+      const float4 x = v[0], y = v[1];
+      q[j] = half8_t{_Float16(x.x), _Float16(x.y), _Float16(x.z), _Float16(x.w),
+                     _Float16(y.x), _Float16(y.y), _Float16(y.z), _Float16(y.w)};
     }
   }
   __device__ __forceinline__ void fetch(const SearchArgs& a, uint32_t rid, int tp, uint4 (&x)[N]) const {
@@ -405,9 +376,18 @@ __device__ __forceinline__ void rerank_list(uint64_t (&top)[E], bool lead, uint3
   if (lead) wave_sort_e<E>(top);
 }
 
-// The query as given into LDS (kBigDim floats, zero past d).
-__device__ __forceinline__ void stage_query(const SearchArgs& a, const float* qsrc, float* s_q, int threads) {
-  for (int i = threadIdx.x; i < kBigDim; i += threads) s_q[i] = masked(qsrc[i < a.d ? i : a.d - 1], i < a.d);
+// The query into LDS, kBigDim floats, zero past d: as given into s_q, and for
+// fp16 traversal centred and scaled as the traversal copy is (its distances
+// are scale^2 times the squared distance) into s_c.
+template <bool F16>
+__device__ __forceinline__ void stage_query(const SearchArgs& a, const float* qsrc, float* s_q, float* s_c,
+                                            int threads) {
+  for (int i = threadIdx.x; i < kBigDim; i += threads) {
+    const int c = i < a.d ? i : int(a.d - 1);
+    const float x = qsrc[c];
+    s_q[i] = masked(x, i < a.d);
+    if constexpr (F16) s_c[i] = masked((x - a.mu[c]) * a.scale, i < a.d);
+  }
 }
 
 // One workgroup of W waves per query.  Wave 0 (the lead wave) owns the
@@ -429,7 +409,7 @@ __global__ __launch_bounds__(64 * W, (F16 && W == 2 && !BIG) ? 4 : 1) void cagra
   const int hcap = bitmap ? (1 << 30) : H / 2;  // a bitmap is never cleared
   const uint32_t hempty = bitmap ? 0u : kInvalidId;
   uint32_t* s_hash = s_mem;
-  uint32_t* s_ids = s_mem + H;                           // 64 fresh ids
+  uint32_t* s_ids = s_mem + (BIG || H > kBigDim ? H : kBigDim);  // 64 fresh ids
   float* s_dist = reinterpret_cast<float*>(s_ids + 64);  // their distances
   uint32_t* s_par = s_ids + 128;                         // parents of this iteration
   // Control words written by the lead wave and read by all after a barrier:
@@ -453,6 +433,17 @@ __global__ __launch_bounds__(64 * W, (F16 && W == 2 && !BIG) ? 4 : 1) void cagra
   const int tm = int(blockIdx.x - qi * a.teams);
   const int team = tid >> 4, tp = lane & 15;
 
+  const float* qsrc = a.queries + qi * a.d;
+  Slice<F16> slice;  // d <= 1024
+  if constexpr (!BIG) {
+    // Staged where the visited set will be (at least kBigDim words); fp16
+    // traversal keeps the query as given in s_q for the final re-rank.
+    float* const staged = reinterpret_cast<float*>(s_mem);
+    stage_query<F16>(a, qsrc, F16 ? s_q : staged, staged, kThreads);
+    __syncthreads();
+    slice.load(staged, tp);
+    __syncthreads();
+  }
   for (int i = tid; i < H; i += kThreads) s_hash[i] = hempty;
   if constexpr (BIG) {
     const float* qg = a.queries + qi * a.d;
@@ -462,10 +453,6 @@ __global__ __launch_bounds__(64 * W, (F16 && W == 2 && !BIG) ? 4 : 1) void cagra
       if (F16) s_qc[i] = i < a.d ? (v - a.mu[i]) * a.scale : 0.f;
     }
   }
-
-  const float* qsrc = a.queries + qi * a.d;
-  Slice<F16> slice;  // d <= 1024
-  if constexpr (!BIG) slice.load(a, qsrc, tp);
 
   // Squared distance of row rid to the query, summed over the 16 lanes of
   // this lane's team: from the traversal copy, or (exact) from the fp32 rows.
@@ -673,7 +660,6 @@ __global__ __launch_bounds__(64 * W, (F16 && W == 2 && !BIG) ? 4 : 1) void cagra
   }
 
   if constexpr (F16) {
-    if constexpr (!BIG) stage_query(a, qsrc, s_q, kThreads);  // published by the re-rank's first barrier
     rerank_list<E, W>(top, lead, s_ids, s_dist, [&](uint32_t rid) { return team_dist(rid, true); });
   }
   if (lead) write_list<E>(a, top, qi, evals, it);
@@ -906,8 +892,15 @@ __global__ __launch_bounds__(64 * W, 2) void cagra_ahead_kernel(SearchArgs a, in
   for (int i = tid; i < kAheadHash; i += kThreads) s_hid[i] = kInvalidId;
   if (tid < 16) s_ctl[tid] = 0u;
   Slice<F16> slice;
-  slice.load(a, qsrc, tp);
-  if constexpr (F16) stage_query(a, qsrc, s_q, kThreads);
+  {
+    // Staged where the entries' keys will be, two barriers on; fp16 traversal
+    // keeps the query as given in s_q for the final re-rank.
+    static_assert(kIds * 2 >= kBigDim, "room for a query");
+    float* const staged = reinterpret_cast<float*>(s_key);
+    stage_query<F16>(a, qsrc, F16 ? s_q : staged, staged, kThreads);
+    __syncthreads();
+    slice.load(staged, tp);
+  }
 
   // Distances of the rows s_ids[0..nf) into s_dist, two rows in flight per team.
   auto evaluate = [&](int nf) {
@@ -1423,6 +1416,7 @@ void cagra_search_device(cvs_context* ctx, const cvs_cagra_index* idx, const flo
   const int64_t bitmap_words = (idx->n + 2047) / 2048 * 64;
   const bool use_bitmap = bitmap_words <= (int64_t(1) << hash_bits);
   const size_t visit_words = use_bitmap ? size_t(bitmap_words) : (size_t(1) << hash_bits);
+  // (The visited set's words hold the query first, see cagra_search_kernel.)
   // Small batches gather for several entries at a time (cagra_ahead_kernel)
   // where that is the faster way.  It pays once the list is long enough that
   // most expansions are of entries already in it: at N=100K D=1024 fp32,
@@ -1440,7 +1434,7 @@ void cagra_search_device(cvs_context* ctx, const cvs_cagra_index* idx, const flo
       itopk > (waves == 8 ? 32 : 64))
     ahead = std::max(itopk > 64 ? kAhead : 6, int(width));
   const bool f16 = idx->traversal_bits == 16;
-  size_t lds = visit_words * 4 + (64 + 64 + CVS_CAGRA_MAX_WIDTH + 8) * 4 +
+  size_t lds = (big ? visit_words : std::max<size_t>(visit_words, kBigDim)) * 4 + (64 + 64 + CVS_CAGRA_MAX_WIDTH + 8) * 4 +
                (big ? size_t(idx->dpad) * 4 * (f16 ? 2 : 1) : (f16 ? size_t(kBigDim) * 4 : 0));
   if (ahead > 0)  // the kernel's arrays, in its order
     lds = visit_words * 4 + size_t(kAhead * 64) * 16 + size_t(kAheadHash) * 8 + (4 * kAhead + 16) * 4 +
