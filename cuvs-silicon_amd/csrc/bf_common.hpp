@@ -25,6 +25,46 @@ constexpr uint64_t kSentinel = ~0ull;
 constexpr int kRsrcWord3 = 0x00020000;
 constexpr int kAuxNT = 2;
 
+using rsrc4 = int __attribute__((ext_vector_type(4)));
+
+// Buffer load straight to LDS (buffer_load ... lds): lane l writes kBytes at
+// LDS byte address m0 + kBytes * l (m0 the same for every lane).  Written as
+// inline assembly so that the compiler does not wait for every outstanding
+// load before each later LDS read (it cannot tell which LDS bytes the load
+// writes); the kernel orders these loads and the reads of their data with
+// explicit s_waitcnt vmcnt and barriers.  M0 is an input operand, so the
+// compiler knows it changes; one wait state separates its write from the
+// load that reads it.
+template <int kBytes, bool kNT>
+__device__ CVS_INLINE void lds_dma(rsrc4 rs, int m0, uint32_t voff, int soff) {
+  if constexpr (kBytes == 16 && kNT)
+    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen nt lds"
+                 :: "v"(voff), "s"(rs), "s"(soff), "{m0}"(m0) : "memory");
+  else if constexpr (kBytes == 16)
+    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+                 :: "v"(voff), "s"(rs), "s"(soff), "{m0}"(m0) : "memory");
+  else
+    asm volatile("s_nop 0\n\tbuffer_load_dword %0, %1, %2 offen lds"
+                 :: "v"(voff), "s"(rs), "s"(soff), "{m0}"(m0) : "memory");
+}
+
+// Raw buffer descriptor: 48-bit base, stride 0, num_records bytes.
+__device__ CVS_INLINE rsrc4 make_rsrc(const void* base, int bytes) {
+  const uint64_t b = reinterpret_cast<uint64_t>(base);
+  rsrc4 r;
+  r.x = int(uint32_t(b));
+  r.y = int(uint32_t(b >> 32) & 0xFFFFu);
+  r.z = bytes;
+  r.w = kRsrcWord3;
+  return r;
+}
+
+// LDS byte address of p, in a scalar register.
+__device__ CVS_INLINE int lds_addr(const void* p) {
+  return __builtin_amdgcn_readfirstlane(
+      int(uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)p))));
+}
+
 enum { kModeScan = 0, kModeSample = 1 };
 
 // List geometry per kp.  Each (workgroup, query) list is split into two
@@ -160,33 +200,70 @@ enum { kCertPass = 0, kCertKeys = 1, kCertAll = 2 };
 // fixed: per lane, float4 partial sums over its 4-column pieces of 256-column
 // chunks, then a butterfly, so a row always gets the same value.  All row
 // loads of a 1024-column pass are issued before the first is used.
+// Up to 128 columns the upper 32 lanes would add zeros: there each half of
+// the wave takes a row of its own, for the same sums.
+__device__ __forceinline__ float sum_sq4(const float4& a, const float4& b) {
+  const float t0 = a.x - b.x, t1 = a.y - b.y, t2 = a.z - b.z, t3 = a.w - b.w;
+  return __fadd_rn(__builtin_fmaf(t1, t1, __fmul_rn(t0, t0)), __builtin_fmaf(t3, t3, __fmul_rn(t2, t2)));
+}
+
+// One pass over NC chunks of 256 columns from column i0 (this lane's first).
+template <int U, int NC>
+__device__ __forceinline__ void exact_chunks(const uint32_t (&id)[U], const float* __restrict__ rows, int64_t n,
+                                             int64_t d, const float* __restrict__ qv, int64_t i0, float (&acc)[U]) {
+  float4 a4[NC], b4[NC][U];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int64_t i = i0 + c * 256;
+    a4[c] = i < d ? *reinterpret_cast<const float4*>(qv + i) : float4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      b4[c][u] = (i < d && int64_t(id[u]) < n) ? *reinterpret_cast<const float4*>(rows + int64_t(id[u]) * d + i)
+                                               : float4{0.f, 0.f, 0.f, 0.f};
+  }
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int u = 0; u < U; ++u) acc[u] = __fadd_rn(acc[u], sum_sq4(a4[c], b4[c][u]));
+}
+
 template <int U>
 __device__ __forceinline__ void wave_exact(const uint32_t (&id)[U], const float* __restrict__ rows, int64_t n,
                                            int64_t d, const float* __restrict__ qv, bool vec, float (&out)[U]) {
+  static_assert(U % 2 == 0, "rows in pairs");
   const int lane = threadIdx.x & 63;
+  if (vec && d <= 128) {
+    uint32_t mine[U / 2];
+    float acc[U / 2];
+#pragma unroll
+    for (int u = 0; u < U / 2; ++u) {
+      mine[u] = lane < 32 ? id[2 * u] : id[2 * u + 1];
+      acc[u] = 0.f;
+    }
+    exact_chunks<U / 2, 1>(mine, rows, n, d, qv, int64_t(lane & 31) * 4, acc);
+#pragma unroll
+    for (int u = 0; u < U / 2; ++u) {
+#pragma unroll
+      for (int o = 16; o >= 1; o >>= 1) acc[u] += xor_lanes_f(acc[u], o);
+      out[2 * u] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(acc[u]), 0));
+      out[2 * u + 1] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(acc[u]), 32));
+    }
+    return;
+  }
   float acc[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) acc[u] = 0.f;
   if (vec) {
-    for (int64_t i0 = int64_t(lane) * 4; i0 < d; i0 += 4 * 256) {
-      float4 a4[4], b4[4][U];
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const int64_t i = i0 + c * 256;
-        a4[c] = i < d ? *reinterpret_cast<const float4*>(qv + i) : float4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-          b4[c][u] = (i < d && int64_t(id[u]) < n) ? *reinterpret_cast<const float4*>(rows + int64_t(id[u]) * d + i)
-                                                   : float4{0.f, 0.f, 0.f, 0.f};
-      }
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const float t0 = a4[c].x - b4[c][u].x, t1 = a4[c].y - b4[c][u].y;
-          const float t2 = a4[c].z - b4[c][u].z, t3 = a4[c].w - b4[c][u].w;
-          acc[u] += (t0 * t0 + t1 * t1) + (t2 * t2 + t3 * t3);
-        }
+    for (int64_t c0 = 0; c0 < d; c0 += 4 * 256) {
+      const int64_t i0 = c0 + int64_t(lane) * 4;
+      if (d - c0 > 768)
+        exact_chunks<U, 4>(id, rows, n, d, qv, i0, acc);
+      else if (d - c0 > 512)
+        exact_chunks<U, 3>(id, rows, n, d, qv, i0, acc);
+      else if (d - c0 > 256)
+        exact_chunks<U, 2>(id, rows, n, d, qv, i0, acc);
+      else
+        exact_chunks<U, 1>(id, rows, n, d, qv, i0, acc);
     }
   } else {
     // Rows that are not 16-byte aligned: one column per lane and load.  The
@@ -293,6 +370,34 @@ GemmPlan plan_gemm_scan(int ks, int kp, int64_t n_rt, int n_qtiles, int compute_
 // Launches it on the context stream; e0 / e1 (may be null) record the
 // dispatch's start and end.
 void launch_gemm_scan(cvs_context* ctx, const GemmArgs& args, int n_wg, hipEvent_t e0, hipEvent_t e1);
+
+// Arguments of the large-batch scan over narrow rows (bf_batch.hip).  Its
+// candidate lists are global for every kp: part[q][range][2 * batch_half(kp)],
+// first kp valid at the end.
+constexpr int batch_half(int kp) { return kp / 2 + 32; }
+constexpr int kBatchMaxRanges = 128;
+struct BatchArgs {
+  const u32x4* tiles;   // dataset tiles
+  const float* norms;   // dataset norms, 32 per tile
+  int64_t n_tiles;
+  const u32x4* qtiles;  // query tiles
+  const float* qnorms;  // query norms, 32 per query tile
+  int nq;
+  int n_qtiles;
+  const float* thr0;    // per-query initial threshold
+  uint64_t* part;
+  uint64_t* lmin;       // [nq][n_ranges] smallest key of each list
+  float* lcut;          // [nq][n_ranges] final threshold of each list
+  int n_ranges;
+  int n_qblocks;
+};
+struct BatchPlan {
+  bool ok = false;      // false: not a padded dimension it handles
+  int n_ranges = 0;     // candidate lists per query
+  int n_qblocks = 0;
+};
+BatchPlan plan_batch_scan(int ks, int64_t q, int64_t n_tiles, int compute_units);
+void launch_batch_scan(cvs_context* ctx, const BatchArgs& args, int ks, int kp, hipEvent_t e0, hipEvent_t e1);
 
 }  // namespace bf
 }  // namespace cvs

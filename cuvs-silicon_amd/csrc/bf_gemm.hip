@@ -68,40 +68,6 @@ using GL = Lists<kKP, kModeScan>;
 // bits 15:14, expcnt in 6:4, lgkmcnt in 11:8; 7 and 15 mean "no wait".
 constexpr int waitcnt_imm(int vm, int lgkm) { return (vm & 0xF) | ((vm >> 4) << 14) | (7 << 4) | (lgkm << 8); }
 
-using rsrc4 = int __attribute__((ext_vector_type(4)));
-
-// Buffer load straight to LDS (buffer_load ... lds): lane l writes kBytes at
-// LDS byte address m0 + kBytes * l (m0 the same for every lane).  Written as
-// inline assembly so that the compiler does not wait for every outstanding
-// load before each later LDS read (it cannot tell which LDS bytes the load
-// writes); the kernel orders these loads and the reads of their data with
-// explicit s_waitcnt vmcnt and barriers.  M0 is an input operand, so the
-// compiler knows it changes; one wait state separates its write from the
-// load that reads it.
-template <int kBytes, bool kNT>
-__device__ CVS_INLINE void lds_dma(rsrc4 rs, int m0, uint32_t voff, int soff) {
-  if constexpr (kBytes == 16 && kNT)
-    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen nt lds"
-                 :: "v"(voff), "s"(rs), "s"(soff), "{m0}"(m0) : "memory");
-  else if constexpr (kBytes == 16)
-    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
-                 :: "v"(voff), "s"(rs), "s"(soff), "{m0}"(m0) : "memory");
-  else
-    asm volatile("s_nop 0\n\tbuffer_load_dword %0, %1, %2 offen lds"
-                 :: "v"(voff), "s"(rs), "s"(soff), "{m0}"(m0) : "memory");
-}
-
-// Raw buffer descriptor: 48-bit base, stride 0, num_records bytes.
-__device__ CVS_INLINE rsrc4 make_rsrc(const void* base, int bytes) {
-  const uint64_t b = reinterpret_cast<uint64_t>(base);
-  rsrc4 r;
-  r.x = int(uint32_t(b));
-  r.y = int(uint32_t(b >> 32) & 0xFFFFu);
-  r.z = bytes;
-  r.w = kRsrcWord3;
-  return r;
-}
-
 __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(1, 1)))
 void bf_gemm_scan_kernel(GemmArgs a) {
   // Stage buffers: 3 x 32 KiB of query tiles, 6 x 8 KiB of row tiles, and
@@ -161,10 +127,6 @@ void bf_gemm_scan_kernel(GemmArgs a) {
   // becomes zero-length past the last stage.  The loads go straight to LDS
   // (buffer_load ... lds: lane l of a wave writes at M0 + size * l): per
   // stage 8 query loads, 2 row loads and 1 norm load per thread.
-  auto lds_addr = [](const void* p) CVS_INLINE {
-    return __builtin_amdgcn_readfirstlane(
-        int(uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)p))));
-  };
   const int q_lds0 = lds_addr(&s_q[0][wave * 64]);
   const int r_lds0 = lds_addr(&s_r[0][wave * 64]);
   const int n_lds0 = lds_addr(&s_norm[0][wave * 64]);

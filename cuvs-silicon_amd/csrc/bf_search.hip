@@ -941,7 +941,8 @@ template <int E>
 __global__ __launch_bounds__(256) void bf_merge_filter_kernel(const uint64_t* __restrict__ part,
                                                               const uint64_t* __restrict__ lmin,
                                                               const float* __restrict__ lcut, int G, int kp,
-                                                              const float* __restrict__ rows, int64_t n, int64_t d,
+                                                              int stride, const float* __restrict__ rows, int64_t n,
+                                                              int64_t d,
                                                               const float* __restrict__ queries, int64_t k,
                                                               Cert cert, uint32_t* __restrict__ out_nbr,
                                                               float* __restrict__ out_dist) {
@@ -954,8 +955,10 @@ __global__ __launch_bounds__(256) void bf_merge_filter_kernel(const uint64_t* __
   __shared__ uint32_t s_cid[64 * E];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t q = blockIdx.x;
-  const uint64_t* src = part + q * int64_t(G) * kp;
+  const uint64_t* src = part + q * int64_t(G) * stride;
   const int total = G * kp;
+  const int lkp = __builtin_ctz(kp);  // kp is a power of two
+  auto entry = [&](int e) { return (e >> lkp) * stride + (e & (kp - 1)); };
   const int R = 2 * kp < 64 * E ? 2 * kp : 64 * E;
   if (tid == 0) s_npass = 0;
 
@@ -985,7 +988,7 @@ __global__ __launch_bounds__(256) void bf_merge_filter_kernel(const uint64_t* __
 #pragma unroll
   for (int r = 0; r < kBatch; ++r) {
     const int e = r * kThreads + tid;
-    key[r] = e < total ? src[e] : kSentinel;
+    key[r] = e < total ? src[entry(e)] : kSentinel;
   }
   if (wave == 0) {
 #pragma unroll
@@ -1022,7 +1025,7 @@ __global__ __launch_bounds__(256) void bf_merge_filter_kernel(const uint64_t* __
 #pragma unroll
       for (int r = 0; r < kBatch; ++r) {
         const int e = b0 + r * kThreads + tid;
-        key[r] = e < total ? src[e] : kSentinel;
+        key[r] = e < total ? src[entry(e)] : kSentinel;
       }
     }
     uint64_t m[kBatch];
@@ -1073,7 +1076,7 @@ __global__ __launch_bounds__(256) void bf_merge_filter_kernel(const uint64_t* __
     }
   }
   __syncthreads();
-  finish_query<E>(s_cid, R, s_tcert, s_tstar, s_keyr, src, G, kp, kp, rows, n, d, queries + q * d, q, k, cert,
+  finish_query<E>(s_cid, R, s_tcert, s_tstar, s_keyr, src, G, kp, stride, rows, n, d, queries + q * d, q, k, cert,
                   out_nbr, out_dist);
 }
 
@@ -1082,14 +1085,75 @@ __global__ __launch_bounds__(256) void bf_merge_filter_kernel(const uint64_t* __
 // R = 64 E smallest keys are the candidates.
 //  1. The R-th smallest list minimum bounds the R-th smallest key (R list
 //     minima are R distinct keys): only keys at or below it can be among
-//     the R smallest.  Each wave computes it (a 256-key wave sort).
-//  2. Each wave streams a quarter of the lists, 64 keys per row, all rows of
-//     a batch loaded at once; a row holding a key within the bound is sorted
-//     (wave bitonic) and merged into the wave's running sorted top-64*E,
-//     whose R-th key then tightens the wave's bound.
-//  3. Wave 0 merges the four running lists; the R candidates are finished
-//     (re-ranked, certified) by finish_query.
+//     the R smallest.  Each wave computes it (a 256-key wave sort) where
+//     there are that many lists.
+//  2. The four waves gather the keys within the bound into LDS, and a radix
+//     select (8 bits a pass, one LDS atomic per key and pass) finds the R-th
+//     smallest; the keys up to it are the candidates, in any order.  (Sorting
+//     the lists 64 keys at a time into running lists took 22,000 of the
+//     56,000 vector instructions of a query at 25 lists; most of the others
+//     were the re-rank's columns past d = 128.  10,000 queries, K = 100:
+//     1M x 128 1.38 -> 0.89 ms, 1M x 1024 1.85 -> 1.79 ms (re-ranked rows: 10.5 GB).)
+//  2b. More keys within the bound than LDS holds (lists that the sampled
+//     threshold did not shorten): each wave streams a quarter of the lists, 64
+//     keys per row, and merges rows holding a key within its bound into its
+//     running sorted top-64*E, whose R-th key tightens the bound; wave 0
+//     merges the four.
+//  3. The candidates are finished (re-ranked, certified) by finish_query.
 // ---------------------------------------------------------------------------
+
+// The need-th smallest (1-based) of the values `v` whose bits above `shift0`
+// + 8 equal those of `pre`, by 8-bit digits from bit shift0 down to 0, over
+// the 256 threads' arrays (count `cnt` of them valid per thread); `need`
+// becomes its rank among the values equal to the result.  s_hist: 256 words.
+template <int M>
+__device__ __forceinline__ uint32_t block_select(const uint32_t (&v)[M], const bool (&ok)[M], int& need,
+                                                 uint32_t* s_hist, int* s_res) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  uint32_t pre = 0;
+  for (int shift = 24; shift >= 0; shift -= 8) {
+    s_hist[tid] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < M; ++i)
+      if (ok[i] && (shift == 24 || ((v[i] ^ pre) >> (shift + 8)) == 0)) atomicAdd(&s_hist[(v[i] >> shift) & 255u], 1u);
+    __syncthreads();
+    if (tid < 64) {
+      // Lane l holds bins 4 l .. 4 l + 3; an inclusive scan over the lanes.
+      const uint4 h = reinterpret_cast<const uint4*>(s_hist)[lane];
+      const uint32_t own = h.x + h.y + h.z + h.w;
+      uint32_t sum = own;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = uint32_t(__shfl_up(int(sum), o));
+        sum += lane >= o ? y : 0u;
+      }
+      const uint32_t before = sum - own;
+      if (before < uint32_t(need) && uint32_t(need) <= sum) {  // exactly one lane
+        uint32_t b = before, bin = 4 * lane;
+        if (b + h.x < uint32_t(need)) {
+          b += h.x;
+          ++bin;
+          if (b + h.y < uint32_t(need)) {
+            b += h.y;
+            ++bin;
+            if (b + h.z < uint32_t(need)) {
+              b += h.z;
+              ++bin;
+            }
+          }
+        }
+        s_res[0] = int(bin);
+        s_res[1] = need - int(b);
+      }
+    }
+    __syncthreads();
+    pre |= uint32_t(s_res[0]) << shift;
+    need = s_res[1];
+  }
+  return pre;
+}
+
 template <int E>
 __global__ __launch_bounds__(256) void bf_merge_kernel(const uint64_t* __restrict__ part,
                                                        const uint64_t* __restrict__ lmin,
@@ -1099,13 +1163,18 @@ __global__ __launch_bounds__(256) void bf_merge_kernel(const uint64_t* __restric
                                                        uint32_t* __restrict__ out_nbr,
                                                        float* __restrict__ out_dist) {
   constexpr int kBatch = 16;
-  __shared__ uint64_t s_run[kWaves][64 * E];
+  constexpr int kMaxPass = kThreads * kBatch;  // gathered keys: one batch per thread
+  __shared__ __attribute__((aligned(16))) uint64_t s_pass[kMaxPass > kWaves * 64 * E ? kMaxPass : kWaves * 64 * E];
+  __shared__ __attribute__((aligned(16))) uint32_t s_hist[256];
   __shared__ uint32_t s_cid[64 * E];
   __shared__ float s_tcert;
   __shared__ uint64_t s_keyr;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  __shared__ uint32_t s_npass, s_ncid;
+  __shared__ int s_res[2];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t q = blockIdx.x;
   constexpr int R = 64 * E;  // candidates re-ranked (>= kp)
+  if (tid == 0) s_npass = s_ncid = 0;
 
   // 1. Bound from the list minima (G <= 256), and the smallest list threshold.
   // Loads unconditional (index clamped; values past G masked to the sentinel
@@ -1124,55 +1193,135 @@ __global__ __launch_bounds__(256) void bf_merge_kernel(const uint64_t* __restric
   }
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) cut = fminf(cut, xor_lanes_f(cut, o));
-  wave_sort_e<4>(mins);
-  uint64_t bound = key_at<4>(mins, R - 1);
+  uint64_t bound = kSentinel;
+  if (G >= R) {
+    wave_sort_e<4>(mins);
+    bound = key_at<4>(mins, R - 1);
+  }
+  __syncthreads();  // the counts are zero
 
-  // 2. This wave's quarter of the 64-key rows.
-  uint64_t run[E];
-#pragma unroll
-  for (int e = 0; e < E; ++e) run[e] = kSentinel;
+  // 2. Gather the keys within the bound.
   const uint64_t* src = part + q * int64_t(G) * stride;
   const int total = G * kp;
-  const int n_rows = (total + 63) / 64;
-  const int r0 = (n_rows * wave) / kWaves, r1 = (n_rows * (wave + 1)) / kWaves;
-  for (int rb = r0; rb < r1; rb += kBatch) {
+  const int lkp = __builtin_ctz(kp);  // kp is a power of two
+  for (int b0 = 0; b0 < total; b0 += kBatch * kThreads) {
     uint64_t key[kBatch];
 #pragma unroll
     for (int r = 0; r < kBatch; ++r) {
-      const int e = (rb + r) * 64 + lane;
-      key[r] = (rb + r < r1 && e < total) ? src[int64_t(e / kp) * stride + e % kp] : kSentinel;
+      const int e = b0 + r * kThreads + tid;
+      key[r] = e < total ? src[int64_t(e >> lkp) * stride + (e & (kp - 1))] : kSentinel;
+    }
+    uint64_t m[kBatch];
+    uint32_t tot = 0;
+#pragma unroll
+    for (int r = 0; r < kBatch; ++r) {
+      m[r] = __ballot(key[r] <= bound && key[r] != kSentinel);
+      tot += uint32_t(popc(m[r]));
+    }
+    if (tot == 0) continue;
+    uint32_t base = 0;
+    if (lane == 0) base = atomicAdd(&s_npass, tot);
+    base = uint32_t(__builtin_amdgcn_readfirstlane(int(base)));
+#pragma unroll
+    for (int r = 0; r < kBatch; ++r) {
+      const uint32_t slot = base + uint32_t(mbcnt(m[r]));
+      if (((m[r] >> lane) & 1ull) && slot < uint32_t(kMaxPass)) s_pass[slot] = key[r];
+      base += uint32_t(popc(m[r]));
+    }
+  }
+  __syncthreads();
+  const int np = int(s_npass);
+  if (np <= kMaxPass) {
+    // The R-th smallest of them, distance word first; what is at or below it
+    // is a candidate.
+    uint64_t key[kBatch];
+    uint32_t hi[kBatch];
+    bool ok[kBatch];
+#pragma unroll
+    for (int r = 0; r < kBatch; ++r) {
+      const int e = r * kThreads + tid;
+      ok[r] = e < np;
+      key[r] = ok[r] ? s_pass[e] : kSentinel;
+      hi[r] = uint32_t(key[r] >> 32);
+    }
+    uint64_t kr = kSentinel;  // fewer than R keys: all of them
+    if (np >= R) {
+      int need = R;
+      const uint32_t kh = block_select<kBatch>(hi, ok, need, s_hist, s_res);
+      uint32_t lo[kBatch];
+      bool eq[kBatch];
+#pragma unroll
+      for (int r = 0; r < kBatch; ++r) {
+        lo[r] = uint32_t(key[r]);
+        eq[r] = ok[r] && hi[r] == kh;
+      }
+      kr = (uint64_t(kh) << 32) | block_select<kBatch>(lo, eq, need, s_hist, s_res);
     }
 #pragma unroll
     for (int r = 0; r < kBatch; ++r) {
-      const bool pass = key[r] != kSentinel && key[r] <= bound;
-      if (__ballot(pass) == 0) continue;
-      uint64_t ck[1] = {pass ? key[r] : kSentinel};
-      wave_sort_e<1>(ck);
-      wave_merge<E>(run, ck[0]);
-      const uint64_t kth = key_at<E>(run, R - 1);
-      bound = kth < bound ? kth : bound;
+      const bool in = ok[r] && key[r] <= kr;
+      const uint64_t m = __ballot(in);
+      if (m == 0) continue;
+      uint32_t base = 0;
+      if (lane == 0) base = atomicAdd(&s_ncid, uint32_t(popc(m)));
+      base = uint32_t(__builtin_amdgcn_readfirstlane(int(base)));
+      if (in) s_cid[base + uint32_t(mbcnt(m))] = uint32_t(key[r]);  // keys are distinct: at most R
     }
-  }
-#pragma unroll
-  for (int e = 0; e < E; ++e) s_run[wave][e * 64 + lane] = run[e];
-  __syncthreads();
-
-  // 3. Merge the four running lists; finish the kp candidates.
-  if (wave == 0) {
-#pragma unroll
-    for (int w = 1; w < kWaves; ++w)
-#pragma unroll
-      for (int e = 0; e < E; ++e) wave_merge<E>(run, s_run[w][e * 64 + lane]);
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-      const int pos = e * 64 + lane;
-      s_cid[pos] = run[e] != kSentinel ? uint32_t(run[e]) : 0xffffffffu;
-    }
-    const uint64_t kr = key_at<E>(run, R - 1);
-    const float tr = kr == kSentinel ? INFINITY : unord_f32(uint32_t(kr >> 32));
-    if (lane == 0) {
-      s_tcert = fminf(tr, cut);
+    __syncthreads();
+    for (int i = int(s_ncid) + tid; i < R; i += kThreads) s_cid[i] = 0xffffffffu;
+    __syncthreads();
+    if (tid == 0) {
+      s_tcert = fminf(kr == kSentinel ? INFINITY : unord_f32(uint32_t(kr >> 32)), cut);
       s_keyr = kr;
+    }
+  } else {
+    // 2b. This wave's quarter of the 64-key rows.
+    uint64_t (*s_run)[64 * E] = reinterpret_cast<uint64_t (*)[64 * E]>(s_pass);
+    __syncthreads();  // s_pass is done with
+    uint64_t run[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) run[e] = kSentinel;
+    const int n_rows = (total + 63) / 64;
+    const int r0 = (n_rows * wave) / kWaves, r1 = (n_rows * (wave + 1)) / kWaves;
+    for (int rb = r0; rb < r1; rb += kBatch) {
+      uint64_t key[kBatch];
+#pragma unroll
+      for (int r = 0; r < kBatch; ++r) {
+        const int e = (rb + r) * 64 + lane;
+        key[r] = (rb + r < r1 && e < total) ? src[int64_t(e / kp) * stride + e % kp] : kSentinel;
+      }
+#pragma unroll
+      for (int r = 0; r < kBatch; ++r) {
+        const bool pass = key[r] != kSentinel && key[r] <= bound;
+        if (__ballot(pass) == 0) continue;
+        uint64_t ck[1] = {pass ? key[r] : kSentinel};
+        wave_sort_e<1>(ck);
+        wave_merge<E>(run, ck[0]);
+        const uint64_t kth = key_at<E>(run, R - 1);
+        bound = kth < bound ? kth : bound;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < E; ++e) s_run[wave][e * 64 + lane] = run[e];
+    __syncthreads();
+
+    // 3. Merge the four running lists; finish the kp candidates.
+    if (wave == 0) {
+#pragma unroll
+      for (int w = 1; w < kWaves; ++w)
+#pragma unroll
+        for (int e = 0; e < E; ++e) wave_merge<E>(run, s_run[w][e * 64 + lane]);
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int pos = e * 64 + lane;
+        s_cid[pos] = run[e] != kSentinel ? uint32_t(run[e]) : 0xffffffffu;
+      }
+      const uint64_t kr = key_at<E>(run, R - 1);
+      const float tr = kr == kSentinel ? INFINITY : unord_f32(uint32_t(kr >> 32));
+      if (lane == 0) {
+        s_tcert = fminf(tr, cut);
+        s_keyr = kr;
+      }
     }
   }
   __syncthreads();
@@ -1238,8 +1387,10 @@ struct BfPlan {
   int kp = 0;              // candidates per (dataset range, query)
   unsigned qblocks = 0;    // 128-query blocks
   bool large_batch = false;
+  bool batch = false;      // large batch, 8 to 20 k-steps: bf_batch.hip
   bool gemm = false;       // large batch, kp = 128: the register-blocked scan (bf_gemm.hip)
-  int gemm_wg = 0;         // its workgroups
+  int batch_qblocks = 0;   // bf_batch.hip's query blocks
+  int gemm_wg = 0;         // bf_gemm.hip's workgroups
   int G = 0;               // candidate lists per query: dataset ranges of the streaming scan
   int stride = 0;          // keys per (query, range) list in the workspace
   int64_t s_units = 0, s_stride = 0;  // threshold sample
@@ -1267,8 +1418,10 @@ void validate_bf(cvs_context* ctx, const cvs_dataset* ds, const float* queries, 
 // True when the call runs the fused scan (else the wide path, bf_wide.hip).
 bool fused_shape(const cvs_dataset* ds, int64_t k) { return ds->d <= kFusedMaxDim && k <= kFusedMaxK; }
 
+// With `batch` false, large batches over narrow rows take the other scans,
+// whose lists need less workspace.
 BfPlan plan_bf(cvs_context* ctx, const cvs_dataset* ds, const float* queries, int64_t q, int64_t k,
-               const uint32_t* nbr, const float* dist) {
+               const uint32_t* nbr, const float* dist, bool batch = true) {
   validate_bf(ctx, ds, queries, q, k, nbr, dist);
   if (!fused_shape(ds, k)) fail(CVS_ERR_UNSUPPORTED, "shape outside the fused scan (d <= 1024, k <= 112)");
 
@@ -1289,9 +1442,16 @@ BfPlan plan_bf(cvs_context* ctx, const cvs_dataset* ds, const float* queries, in
   if (global_lists && G > 128) G = 128;
   if (p.large_batch && G > 32) G = 32;
   if (int64_t(G) > p.n_units) G = int(p.n_units);
-  // Large batches with kp = 128 run the register-blocked scan: persistent
-  // workgroups over (query block, row block) units, n_lists lists per query.
-  if (p.large_batch) {
+  // Large batches over narrow rows run bf_batch.hip; other large batches
+  // with kp = 128 the register-blocked scan: persistent workgroups over
+  // (query block, row block) units, n_lists lists per query.
+  BatchPlan bp;
+  if (p.large_batch && batch) bp = plan_batch_scan(p.ks, q, ds->n_tiles, ctx->compute_units);
+  if (bp.ok) {
+    p.batch = true;
+    p.batch_qblocks = bp.n_qblocks;
+    G = bp.n_ranges;
+  } else if (p.large_batch) {
     const GemmPlan gp = plan_gemm_scan(p.ks, p.kp, ds->n_tiles / 4, int((q + 31) / 32), ctx->compute_units);
     if (gp.ok) {
       p.gemm = true;
@@ -1300,10 +1460,11 @@ BfPlan plan_bf(cvs_context* ctx, const cvs_dataset* ds, const float* queries, in
     }
   }
   p.G = G;
-  p.stride = global_lists ? Lists<128, kModeScan>::CAP : p.kp;
+  p.stride = p.batch ? 2 * batch_half(p.kp) : global_lists ? Lists<128, kModeScan>::CAP : p.kp;
 
-  // Sample: 16,384 rows for small batches, 65,536 for other large ones and
-  // 32,768 for the register-blocked scan, in whole units, evenly strided,
+  // Sample: 16,384 rows for small batches, 65,536 for large ones of the
+  // streaming scan and 32,768 for the two large-batch scans (bf_batch.hip:
+  // 65,536 rows cost 240 us more at 10,000 queries and save as much), evenly strided,
   // over Gs workgroups; 2 minima per (query, workgroup).  The initial
   // threshold (below) then sits near rank r * n / sample of each query's
   // distances, so a workgroup's lists see about r * n / (sample * G)
@@ -1313,7 +1474,7 @@ BfPlan plan_bf(cvs_context* ctx, const cvs_dataset* ds, const float* queries, in
   // and compactions sit on its critical path, so its threshold rank matters
   // (about 2 ms per doubling at N=1M Q=10,000 K=100); with the rank rule
   // below a 32,768-row sample keeps it at ~977 for 1.15 ms of sampling.
-  p.s_units = (p.gemm ? 32768 : p.large_batch ? 65536 : 16384) / rpu;
+  p.s_units = (p.gemm || p.batch ? 32768 : p.large_batch ? 65536 : 16384) / rpu;
   if (p.s_units < 1) p.s_units = 1;
   if (p.s_units > p.n_units) p.s_units = p.n_units;
   p.s_stride = p.n_units / p.s_units;
@@ -1413,7 +1574,23 @@ void bf_launch(cvs_context* ctx, const cvs_dataset* ds, const BfPlan& p, const f
   after_launch("bf_select_kernel");
 
   const TimerSpan t2 = timed ? timer_span(ctx, "bf_scan") : TimerSpan{};
-  if (p.gemm) {
+  if (p.batch) {
+    BatchArgs ba{};
+    ba.tiles = args.tiles;
+    ba.norms = ds->norms;
+    ba.n_tiles = ds->n_tiles;
+    ba.qtiles = qtiles;
+    ba.qnorms = qnorms;
+    ba.nq = int(q);
+    ba.n_qtiles = int(p.q_tiles);
+    ba.thr0 = thr0;
+    ba.part = part;
+    ba.lmin = lmin;
+    ba.lcut = lcut;
+    ba.n_ranges = G;
+    ba.n_qblocks = p.batch_qblocks;
+    launch_batch_scan(ctx, ba, p.ks, kp, t2.start, t2.stop);
+  } else if (p.gemm) {
     GemmArgs ga{};
     ga.tiles = args.tiles;
     ga.norms = ds->norms;
@@ -1446,13 +1623,13 @@ void bf_launch(cvs_context* ctx, const cvs_dataset* ds, const BfPlan& p, const f
   if (kp <= 32)
     hipExtLaunchKernelGGL(bf_merge_filter_kernel<1>, dim3(unsigned(q)), dim3(kThreads), 0, ctx->stream, t3.start,
                           t3.stop, 0, static_cast<const uint64_t*>(part), static_cast<const uint64_t*>(lmin),
-                          static_cast<const float*>(lcut), G, kp, static_cast<const float*>(ds->rows), ds->n, ds->d,
-                          queries, k, cert, nbr, dist);
+                          static_cast<const float*>(lcut), G, kp, p.stride, static_cast<const float*>(ds->rows), ds->n,
+                          ds->d, queries, k, cert, nbr, dist);
   else if (kp <= 64)
     hipExtLaunchKernelGGL(bf_merge_filter_kernel<2>, dim3(unsigned(q)), dim3(kThreads), 0, ctx->stream, t3.start,
                           t3.stop, 0, static_cast<const uint64_t*>(part), static_cast<const uint64_t*>(lmin),
-                          static_cast<const float*>(lcut), G, kp, static_cast<const float*>(ds->rows), ds->n, ds->d,
-                          queries, k, cert, nbr, dist);
+                          static_cast<const float*>(lcut), G, kp, p.stride, static_cast<const float*>(ds->rows), ds->n,
+                          ds->d, queries, k, cert, nbr, dist);
   else
     hipExtLaunchKernelGGL(bf_merge_kernel<4>, dim3(unsigned(q)), dim3(kThreads), 0, ctx->stream, t3.start, t3.stop,
                           0, static_cast<const uint64_t*>(part), static_cast<const uint64_t*>(lmin),
@@ -1553,7 +1730,9 @@ int cvs_bf_search_noalloc(cvs_context* ctx, const cvs_dataset* ds, const float* 
     validate_bf(ctx, ds, queries_dev, q, k, out_neighbors_dev, out_distances_dev);
     if (!fused_shape(ds, k))
       fail(CVS_ERR_UNSUPPORTED, "cvs_bf_search_noalloc runs the fused scan only: d <= 1024 and k <= 112");
-    const BfPlan p = plan_bf(ctx, ds, queries_dev, q, k, out_neighbors_dev, out_distances_dev);
+    BfPlan p = plan_bf(ctx, ds, queries_dev, q, k, out_neighbors_dev, out_distances_dev);
+    if (p.batch && p.total > kScratchBytes)
+      p = plan_bf(ctx, ds, queries_dev, q, k, out_neighbors_dev, out_distances_dev, false);
     if (p.total > kScratchBytes)
       fail(CVS_ERR_UNSUPPORTED, "cvs_bf_search_noalloc: this call needs " + std::to_string(p.total) +
                                     " bytes of scratch, more than the " + std::to_string(kScratchBytes) +

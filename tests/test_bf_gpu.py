@@ -116,6 +116,72 @@ def test_random_shapes(ctx, oracle, n, d, q, k):
     check_against_oracle(ctx, oracle, base, qs, k)
 
 
+@pytest.mark.parametrize("copies,k", [(0, 49), (300, 100), (4000, 112), (9000, 100)])
+@pytest.mark.parametrize("d", [20, 128, 132, 515, 1024])
+def test_merge_of_long_lists(ctx, d, copies, k):
+    """kp = 128: the candidates are selected among the listed keys (equal
+    distances cut by the row id), or, when more keys lie within the bound than
+    the merge's buffer holds (9,000 copies of one row), from running lists.
+    Whole numbers: ids and distances equal those of a sort by (distance, id).
+    The dimensions cover the exact re-rank's forms: half a wave a row, one to
+    four chunks of 256 columns, unaligned rows."""
+    rng = np.random.default_rng(d + copies)
+    n, q = 40_000, 7
+    base = rng.integers(-5, 6, (n, d)).astype(np.float32)
+    base[rng.choice(n, copies, replace=False)] = base[0]
+    qs = np.concatenate([base[:1], rng.integers(-5, 6, (q - 1, d)).astype(np.float32)])
+    nbr, dist = ctx.dataset(base).bf_search(qs, k)
+    key = ((qs.astype(np.float64) ** 2).sum(1)[:, None] - 2.0 * (qs.astype(np.float64) @ base.T.astype(np.float64))
+           + (base.astype(np.float64) ** 2).sum(1)[None, :]).astype(np.int64) * n + np.arange(n)[None, :]
+    near = np.sort(np.partition(key, k - 1, axis=1)[:, :k], axis=1)
+    np.testing.assert_array_equal(nbr, near % n)
+    np.testing.assert_array_equal(dist, near // n)
+
+
+@pytest.mark.parametrize("d", [65, 128, 160, 256, 320])
+@pytest.mark.parametrize("n,q,k", [
+    (2500, 1025, 10),    # one query past the limit; part-filled last workgroup and query tile
+    (20001, 1600, 24),
+    (9000, 1281, 48),
+    (70, 1100, 100),     # k > n, most ranges empty
+    (30000, 1030, 112),
+])
+def test_narrow_large_batches(ctx, d, n, q, k):
+    """The large-batch scan over 8 to 20 k-steps, every list geometry.  Rows
+    in order of falling distance to the queries, so that keys keep passing and
+    lists are compacted; whole numbers, so ids equal those of a sort by
+    (distance, id)."""
+    rng = np.random.default_rng(d + n)
+    base = rng.integers(-6, 7, (n, d)).astype(np.float32)
+    base[:, 0] = np.rint(np.linspace(200, 0, n))
+    qs = rng.integers(-6, 7, (q, d)).astype(np.float32)
+    nbr, dist = ctx.dataset(base).bf_search(qs, k)
+    key = ((qs.astype(np.float64) ** 2).sum(1)[:, None] - 2.0 * (qs.astype(np.float64) @ base.T.astype(np.float64))
+           + (base.astype(np.float64) ** 2).sum(1)[None, :]).astype(np.int64) * n + np.arange(n)[None, :]
+    m = min(k, n)
+    near = np.sort(np.partition(key, m - 1, axis=1)[:, :m], axis=1)
+    np.testing.assert_array_equal(nbr[:, :m], near % n)
+    np.testing.assert_array_equal(dist[:, :m], near // n)
+    assert (nbr[:, m:] == 0xFFFFFFFF).all() and np.isinf(dist[:, m:]).all()
+
+
+@pytest.mark.parametrize("q,k", [(2000, 10), (1100, 24)])
+def test_narrow_large_batches_without_allocation(ctx, cvs, q, k):
+    """The fixed scratch of the allocation-free call is too small for that
+    scan's lists at some sizes it takes: it then runs another scan."""
+    rng = np.random.default_rng(q + k)
+    base = rng.integers(-6, 7, (30_000, 128)).astype(np.float32)
+    qs = rng.integers(-6, 7, (q, 128)).astype(np.float32)
+    ds = ctx.dataset(base)
+    want_nbr, want_dist = ds.bf_search(qs, k)
+    queries = cvs.DeviceArray.from_host(ctx, qs)
+    nbr, dist = cvs.DeviceArray(ctx, (q, k), np.uint32), cvs.DeviceArray(ctx, (q, k), np.float32)
+    ds.bf_search_noalloc(queries, k, nbr, dist)
+    ctx.synchronize()
+    np.testing.assert_array_equal(nbr.to_host(), want_nbr)
+    np.testing.assert_array_equal(dist.to_host(), want_dist)
+
+
 @pytest.mark.parametrize("d", [129, 192, 193, 320, 321, 384, 385, 448, 449, 640, 641, 768, 769, 896, 897])
 @pytest.mark.parametrize("n,q,k", [
     (17000, 33, 10), (9001, 130, 24), (6002, 5, 48), (4003, 20, 100),  # one list geometry each
