@@ -1751,16 +1751,8 @@ int cvs_bf_search(cvs_context* ctx, const cvs_dataset* ds, const float* queries,
     if (q <= 0 || k <= 0) fail(CVS_ERR_INVALID_ARGUMENT, "query count and k must be positive");
     const size_t qbytes = size_t(q) * size_t(ds->d) * sizeof(float);
     const size_t obytes = size_t(q) * size_t(k) * sizeof(float);
-    ctx->ws_io.reserve(qbytes + 2 * obytes + 256);
-    char* base = ctx->ws_io.as<char>();
-    float* dq = reinterpret_cast<float*>(base);
-    uint32_t* dn = reinterpret_cast<uint32_t*>(base + (qbytes + 127) / 128 * 128);
-    float* dd = reinterpret_cast<float*>(reinterpret_cast<char*>(dn) + (obytes + 127) / 128 * 128);
-    CVS_HIP(hipMemcpyAsync(dq, queries, qbytes, hipMemcpyHostToDevice, ctx->stream));
-    bf_search_device(ctx, ds, dq, q, k, dn, dd);
-    CVS_HIP(hipMemcpyAsync(out_neighbors, dn, obytes, hipMemcpyDeviceToHost, ctx->stream));
-    CVS_HIP(hipMemcpyAsync(out_distances, dd, obytes, hipMemcpyDeviceToHost, ctx->stream));
-    CVS_HIP(hipStreamSynchronize(ctx->stream));
+    host_call(ctx, queries, qbytes, out_neighbors, out_distances, obytes,
+              [&](const float* dq, uint32_t* dn, float* dd) { bf_search_device(ctx, ds, dq, q, k, dn, dd); });
   });
 }
 

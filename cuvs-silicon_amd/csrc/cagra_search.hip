@@ -1728,17 +1728,10 @@ int cvs_cagra_search_teams(cvs_context* ctx, const cvs_cagra_index* index, const
     if (q <= 0 || k <= 0) fail(CVS_ERR_INVALID_ARGUMENT, "query count and k must be positive");
     const size_t qbytes = size_t(q) * size_t(index->d) * sizeof(float);
     const size_t obytes = size_t(q) * size_t(k) * sizeof(float);
-    ctx->ws_io.reserve(qbytes + 2 * obytes + 256);
-    char* base = ctx->ws_io.as<char>();
-    float* dq = reinterpret_cast<float*>(base);
-    uint32_t* dn = reinterpret_cast<uint32_t*>(base + (qbytes + 127) / 128 * 128);
-    float* dd = reinterpret_cast<float*>(reinterpret_cast<char*>(dn) + (obytes + 127) / 128 * 128);
-    CVS_HIP(hipMemcpyAsync(dq, queries, qbytes, hipMemcpyHostToDevice, ctx->stream));
-    cagra_search_device(ctx, index, dq, q, k, itopk_size, search_width, max_iterations, dn, dd, nullptr,
-                        int(std::min<uint32_t>(teams, 1u << 20)));
-    CVS_HIP(hipMemcpyAsync(out_neighbors, dn, obytes, hipMemcpyDeviceToHost, ctx->stream));
-    CVS_HIP(hipMemcpyAsync(out_distances, dd, obytes, hipMemcpyDeviceToHost, ctx->stream));
-    CVS_HIP(hipStreamSynchronize(ctx->stream));
+    host_call(ctx, queries, qbytes, out_neighbors, out_distances, obytes, [&](const float* dq, uint32_t* dn, float* dd) {
+      cagra_search_device(ctx, index, dq, q, k, itopk_size, search_width, max_iterations, dn, dd, nullptr,
+                          int(std::min<uint32_t>(teams, 1u << 20)));
+    });
   });
 }
 
@@ -1752,16 +1745,9 @@ int cvs_cagra_search(cvs_context* ctx, const cvs_cagra_index* index, const float
     if (q <= 0 || k <= 0) fail(CVS_ERR_INVALID_ARGUMENT, "query count and k must be positive");
     const size_t qbytes = size_t(q) * size_t(index->d) * sizeof(float);
     const size_t obytes = size_t(q) * size_t(k) * sizeof(float);
-    ctx->ws_io.reserve(qbytes + 2 * obytes + 256);
-    char* base = ctx->ws_io.as<char>();
-    float* dq = reinterpret_cast<float*>(base);
-    uint32_t* dn = reinterpret_cast<uint32_t*>(base + (qbytes + 127) / 128 * 128);
-    float* dd = reinterpret_cast<float*>(reinterpret_cast<char*>(dn) + (obytes + 127) / 128 * 128);
-    CVS_HIP(hipMemcpyAsync(dq, queries, qbytes, hipMemcpyHostToDevice, ctx->stream));
-    cagra_search_device(ctx, index, dq, q, k, itopk_size, search_width, max_iterations, dn, dd, nullptr);
-    CVS_HIP(hipMemcpyAsync(out_neighbors, dn, obytes, hipMemcpyDeviceToHost, ctx->stream));
-    CVS_HIP(hipMemcpyAsync(out_distances, dd, obytes, hipMemcpyDeviceToHost, ctx->stream));
-    CVS_HIP(hipStreamSynchronize(ctx->stream));
+    host_call(ctx, queries, qbytes, out_neighbors, out_distances, obytes, [&](const float* dq, uint32_t* dn, float* dd) {
+      cagra_search_device(ctx, index, dq, q, k, itopk_size, search_width, max_iterations, dn, dd, nullptr);
+    });
   });
 }
 

@@ -6,6 +6,7 @@
 
 #include <cstdint>
 #include <cstdio>
+#include <functional>
 #include <map>
 #include <stdexcept>
 #include <string>
@@ -90,6 +91,9 @@ struct cvs_context {
   cvs::DeviceBuffer ws_search;    // brute force: query tiles, thresholds, candidate lists
   cvs::DeviceBuffer ws_io;        // staging of host queries / results
   cvs::DeviceBuffer ws_teams;     // per-team lists of multi-team graph search
+  // Pinned host memory of kPinnedIoBytes for small blocking calls (host_call);
+  // made by the first one.
+  char* pinned_io = nullptr;
   // Brute-force escalation counters (device, allocated with the context):
   // [0] queries whose fp16 selection could not be certified and were
   // re-ranked exactly over more rows, [1] of them over every row.
@@ -195,6 +199,19 @@ inline int64_t padded_dim(int64_t d) {
     if (d <= ks * 16) return ks * 16;
   return 1024;
 }
+
+// A blocking search on host buffers: `run` enqueues it on the context stream
+// given device-visible queries, ids and distances (qbytes, obytes, obytes).
+//
+// Calls that fit kPinnedIoBytes go through pinned memory: a kernel copies the
+// queries from it to the device (the search reads them more than once), and
+// the search's last kernel writes its results straight into it.  The three
+// hipMemcpyAsync of pageable buffers that larger calls use cost about 20 us
+// each, most of it between the copies: one query to 100,000 x 768 took 116 us,
+// 71 now.
+constexpr size_t kPinnedIoBytes = size_t(1) << 20;
+void host_call(cvs_context* ctx, const float* queries, size_t qbytes, uint32_t* nbr, float* dist, size_t obytes,
+               const std::function<void(const float*, uint32_t*, float*)>& run);
 
 // Launches the fp32 -> fp16-tile conversion of scale * (row - mu) (rows n x
 // d with row stride d; mu d floats, or null for zero); writes n_tiles tiles

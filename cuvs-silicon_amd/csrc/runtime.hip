@@ -72,6 +72,53 @@ void upload_rows(cvs_context* ctx, float* dst, int64_t pitch, const float* src, 
   check_hip(e, "hipMemcpy2DAsync");
 }
 
+namespace {
+__global__ __launch_bounds__(256) void copy_in_kernel(const uint4* __restrict__ src, uint4* __restrict__ dst,
+                                                      size_t count) {
+  const size_t i = size_t(blockIdx.x) * 256 + threadIdx.x;
+  if (i < count) dst[i] = src[i];
+}
+}  // namespace
+
+void host_call(cvs_context* ctx, const float* queries, size_t qbytes, uint32_t* nbr, float* dist, size_t obytes,
+               const std::function<void(const float*, uint32_t*, float*)>& run) {
+  const size_t qspan = (qbytes + 127) / 128 * 128, ospan = (obytes + 127) / 128 * 128;
+  if (qspan + 2 * ospan <= kPinnedIoBytes) {
+    if (!ctx->pinned_io)
+      CVS_HIP(hipHostMalloc(reinterpret_cast<void**>(&ctx->pinned_io), kPinnedIoBytes, hipHostMallocDefault));
+    char* const pin = ctx->pinned_io;
+    uint32_t* const pn = reinterpret_cast<uint32_t*>(pin + qspan);
+    float* const pd = reinterpret_cast<float*>(pin + qspan + ospan);
+    ctx->ws_io.reserve(qspan);
+    float* const dq = ctx->ws_io.as<float>();
+    std::memcpy(pin, queries, qbytes);
+    const size_t count = (qbytes + 15) / 16;  // within both spans
+    hipLaunchKernelGGL(copy_in_kernel, dim3(unsigned((count + 255) / 256)), dim3(256), 0, ctx->stream,
+                       reinterpret_cast<const uint4*>(pin), reinterpret_cast<uint4*>(dq), count);
+    CVS_HIP(hipGetLastError());
+    try {
+      run(dq, pn, pd);
+    } catch (...) {
+      (void)hipStreamSynchronize(ctx->stream);  // the pinned memory is free again
+      throw;
+    }
+    CVS_HIP(hipStreamSynchronize(ctx->stream));
+    std::memcpy(nbr, pn, obytes);
+    std::memcpy(dist, pd, obytes);
+    return;
+  }
+  ctx->ws_io.reserve(qspan + 2 * ospan);
+  char* const base = ctx->ws_io.as<char>();
+  float* const dq = reinterpret_cast<float*>(base);
+  uint32_t* const dn = reinterpret_cast<uint32_t*>(base + qspan);
+  float* const dd = reinterpret_cast<float*>(base + qspan + ospan);
+  CVS_HIP(hipMemcpyAsync(dq, queries, qbytes, hipMemcpyHostToDevice, ctx->stream));
+  run(dq, dn, dd);
+  CVS_HIP(hipMemcpyAsync(nbr, dn, obytes, hipMemcpyDeviceToHost, ctx->stream));
+  CVS_HIP(hipMemcpyAsync(dist, dd, obytes, hipMemcpyDeviceToHost, ctx->stream));
+  CVS_HIP(hipStreamSynchronize(ctx->stream));
+}
+
 TimerSpan timer_span(cvs_context* ctx, const char* kernel) {
   if (!ctx->timing) return {};
   KernelTimer& t = ctx->timers[kernel];
@@ -493,6 +540,7 @@ int cvs_context_destroy(cvs_context* ctx) {
     ctx->ws_search.release();
     ctx->ws_io.release();
     ctx->ws_teams.release();
+    if (ctx->pinned_io) (void)hipHostFree(ctx->pinned_io);
     if (ctx->bf_counters) (void)hipFree(ctx->bf_counters);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;

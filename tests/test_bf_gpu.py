@@ -116,6 +116,26 @@ def test_random_shapes(ctx, oracle, n, d, q, k):
     check_against_oracle(ctx, oracle, base, qs, k)
 
 
+@pytest.mark.parametrize("q", [1, 250, 252])
+def test_blocking_calls_on_both_sides_of_the_pinned_limit(ctx, cvs, q):
+    """250 queries of 1,024 columns with 10 results each fit the pinned
+    staging (1 MiB), 252 do not; a refused call in between leaves nothing
+    behind."""
+    rng = np.random.default_rng(q)
+    base = rng.integers(-6, 7, (3000, 1024)).astype(np.float32)
+    qs = rng.integers(-6, 7, (q, 1024)).astype(np.float32)
+    ds = ctx.dataset(base)
+    with pytest.raises(ValueError):
+        ds.bf_search(qs[:1], 1025)
+    nbr, dist = ds.bf_search(qs, 10)
+    queries = cvs.DeviceArray.from_host(ctx, qs)
+    want_nbr, want_dist = cvs.DeviceArray(ctx, (q, 10), np.uint32), cvs.DeviceArray(ctx, (q, 10), np.float32)
+    ds.bf_search_async(queries, 10, want_nbr, want_dist)
+    ctx.synchronize()
+    np.testing.assert_array_equal(nbr, want_nbr.to_host())
+    np.testing.assert_array_equal(dist, want_dist.to_host())
+
+
 @pytest.mark.parametrize("copies,k", [(0, 49), (300, 100), (4000, 112), (9000, 100)])
 @pytest.mark.parametrize("d", [20, 128, 132, 515, 1024])
 def test_merge_of_long_lists(ctx, d, copies, k):
