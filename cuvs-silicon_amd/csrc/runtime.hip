@@ -83,9 +83,13 @@ __global__ __launch_bounds__(256) void copy_in_kernel(const uint4* __restrict__ 
 void host_call(cvs_context* ctx, const float* queries, size_t qbytes, uint32_t* nbr, float* dist, size_t obytes,
                const std::function<void(const float*, uint32_t*, float*)>& run) {
   const size_t qspan = (qbytes + 127) / 128 * 128, ospan = (obytes + 127) / 128 * 128;
-  if (qspan + 2 * ospan <= kPinnedIoBytes) {
-    if (!ctx->pinned_io)
-      CVS_HIP(hipHostMalloc(reinterpret_cast<void**>(&ctx->pinned_io), kPinnedIoBytes, hipHostMallocDefault));
+  const bool fits = qspan <= kPinnedIoBytes && 2 * ospan <= kPinnedIoBytes - qspan;
+  if (fits && !ctx->pinned_io &&
+      hipHostMalloc(reinterpret_cast<void**>(&ctx->pinned_io), kPinnedIoBytes, hipHostMallocDefault) != hipSuccess) {
+    ctx->pinned_io = nullptr;
+    (void)hipGetLastError();  // no pinned memory to be had: copies
+  }
+  if (fits && ctx->pinned_io) {
     char* const pin = ctx->pinned_io;
     uint32_t* const pn = reinterpret_cast<uint32_t*>(pin + qspan);
     float* const pd = reinterpret_cast<float*>(pin + qspan + ospan);
