@@ -11,12 +11,14 @@
 //  prep     queries fp32 -> fp16 32-row tiles + norms (the dataset layout),
 //           one wave per query.
 //  sample   the scan kernel over an evenly strided sample of 16,384 rows
-//           (65,536 for other large batches, 32,768 when the register-blocked
-//           scan of bf_gemm.hip follows); each lane keeps the minimum distance
+//           (65,536 for other large batches, 32,768 when one of the
+//           large-batch scans of bf_gemm.hip and bf_batch.hip follows); each
+//           lane keeps the minimum distance
 //           of the rows it sees, so every (query, workgroup, half-wave)
 //           yields one minimum.
-//  select   per query (one wave), the r-th smallest of those minima, T0.
-//           The r smallest minima are r distinct dataset rows, so at least r
+//  select   per query (one wave), the r-th smallest of those minima (or, for
+//           small batches, of the lanes' minima of them), T0.  The r
+//           smallest minima are r distinct dataset rows, so at least r
 //           rows lie at or below T0 and every row above it can be dropped by
 //           the scan.  r is set on the host (plan_bf) so that T0 falls below
 //           the merge's R candidates with probability at most 1e-9.
@@ -38,8 +40,8 @@
 //  merge    one workgroup per query: the R-th smallest list minimum bounds
 //           the R-th smallest key (R = 2 kp, at most 256).  For kp <= 64 every
 //           key within it is gathered into LDS and one wave keeps the R
-//           smallest; for kp = 128 each wave merges the 64-key rows holding a
-//           key within the bound into its running top-R.  The R candidates
+//           smallest; for kp = 128 a radix select finds the R-th.  The R
+//           candidates
 //           are re-ranked with exact fp32 distances from the fp32 rows,
 //           sorted by (distance, id), certified against the fp16 error bound
 //           (bf_common.hpp, Cert; a query that fails is re-ranked over more

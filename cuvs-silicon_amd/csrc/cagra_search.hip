@@ -29,6 +29,8 @@
 //    before the sort.
 //  - waves per query: 2 for large batches; 4 or 8 when the batch is small
 //    and each query's chain of dependent gathers is the latency (Q = 1).
+//    Most of those small batches run cagra_ahead_kernel, which shortens that
+//    chain: the rows of several parents gathered in one step.
 //
 // Iteration: pick the first `width` unexpanded entries of the list as
 // parents, mark them, evaluate their neighbours.  Stop when the list holds no
