@@ -700,10 +700,17 @@ __device__ __forceinline__ uint32_t wave_min_u32(uint32_t x) {
 // the test above rejects them as parents and the list is cut to itopk keys at
 // the end.  One wave uses the pool; every member but front and rest is uniform
 // over it.
+constexpr int kAhead = 8;           // entries that one step may expand
+constexpr int kIds = kAhead * 64;   // candidates of one step at most
+
 template <int E>
 struct Pool {
-  static constexpr int kFull = 512;              // buf is emptied at this many keys
-  static constexpr int kBuf = kFull + 128 + 16;  // one add, the parents of one step
+  static constexpr int kFull = 512;  // buf is emptied before a step at this many keys
+  // A step below that adds its parents and all its candidates (a candidate
+  // goes into buf itself or displaces one key of front into it) with no look
+  // at nbuf in between.  Emptying it between two adds instead, with room for
+  // 144 keys, took 1.5% longer (itopk 512 Q=100 816 us, 805 with this room).
+  static constexpr int kBuf = kFull + kAhead + kIds;
   static constexpr int kNear = 65;               // refill: the nearest unexpanded keys and one more
   static constexpr int kLds = kBuf + kNear + 64 * E;
   uint64_t front, rest[E];
@@ -856,14 +863,12 @@ struct Pool {
 // the new candidates, 2,400 the run of iterations and the visited set, 1,900
 // the graph rows: latencies of single instructions of one wave for the most
 // part.
-constexpr int kAhead = 8;         // entries with keys at hand
-constexpr int kAheadHash = 1024;  // ids of one step: at most kAhead * 64, half full
+constexpr int kAheadHash = 2 * kIds;  // ids of one step: at most half full
 
 template <int E, int W, bool F16>
 __global__ __launch_bounds__(64 * W, 2) void cagra_ahead_kernel(SearchArgs a, int ahead) {
   extern __shared__ uint32_t s_mem[];
   constexpr int kThreads = 64 * W, kTeams = 4 * W;
-  constexpr int kIds = kAhead * 64;      // candidates of one step
   constexpr int kPerWave = kAhead / W;   // entries per wave and step
   static_assert(kPerWave * W == kAhead, "entries per wave");
   uint32_t* s_bits = s_mem;                               // visited rows (bitmap_words: whole 256-byte blocks)
@@ -1183,13 +1188,19 @@ int waves_per_query(int64_t workgroups) {
 template <int E, bool F16>
 void launch_search(int waves, bool big, int ahead, dim3 grid, size_t lds, hipStream_t stream, const SearchArgs& a,
                    hipEvent_t e0, hipEvent_t e1) {
-  if (ahead > 0 && waves == 8) {
-    hipExtLaunchKernelGGL((cagra_ahead_kernel<E, 8, F16>), grid, dim3(512), lds, stream, e0, e1, 0, a, ahead);
-    return;
-  }
-  if constexpr (E > 1) {
-    if (ahead > 0) {
-      hipExtLaunchKernelGGL((cagra_ahead_kernel<E, 4, F16>), grid, dim3(256), lds, stream, e0, e1, 0, a, ahead);
+  if (ahead > 0) {
+    auto go = [&](auto kernel, int threads) {
+      if (lds > 64 * 1024)  // fp16 traversal, itopk > 256, more than 253,952 rows
+        CVS_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    int(lds)));
+      hipExtLaunchKernelGGL(kernel, grid, dim3(threads), lds, stream, e0, e1, 0, a, ahead);
+    };
+    if (waves == 8) {
+      go(cagra_ahead_kernel<E, 8, F16>, 512);
+      return;
+    }
+    if constexpr (E > 1) {
+      go(cagra_ahead_kernel<E, 4, F16>, 256);
       return;
     }
   }
@@ -1439,7 +1450,7 @@ void cagra_search_device(cvs_context* ctx, const cvs_cagra_index* idx, const flo
   size_t lds = (big ? visit_words : std::max<size_t>(visit_words, kBigDim)) * 4 + (64 + 64 + CVS_CAGRA_MAX_WIDTH + 8) * 4 +
                (big ? size_t(idx->dpad) * 4 * (f16 ? 2 : 1) : (f16 ? size_t(kBigDim) * 4 : 0));
   if (ahead > 0)  // the kernel's arrays, in its order
-    lds = visit_words * 4 + size_t(kAhead * 64) * 16 + size_t(kAheadHash) * 8 + (4 * kAhead + 16) * 4 +
+    lds = visit_words * 4 + size_t(kIds) * 16 + size_t(kAheadHash) * 8 + (4 * kAhead + 16) * 4 +
           size_t(Pool<1>::kLds + 64 * (e_slots - 1) + 1) * 8 + (f16 ? size_t(kBigDim) * 4 : 0);
 
   SearchArgs a{};

@@ -46,6 +46,17 @@ def search(ctx, cvs, idx, qs, k, knobs):
     (5000, 1024, 64, "knn", 10, 1, 0),       # a list shorter than the parents gathered ahead
     (3000, 128, 32, "random", 300, 4, 7),    # cut off by max_iterations
     (1, 16, 1, "random", 32, 1, 0),
+    # Hundreds of new keys in one step, again and again: the pool's buffer has
+    # to hold up to 999 keys.  Every list length; wide steps and runs of single
+    # parents.
+    (20000, 32, 64, "random", 64, 8, 0),
+    (20000, 32, 64, "random", 128, 4, 0),
+    (20000, 32, 64, "random", 256, 1, 0),
+    (20000, 32, 64, "random", 256, 8, 0),
+    (20000, 32, 64, "random", 512, 1, 0),
+    (20000, 32, 64, "random", 512, 8, 0),
+    (20000, 32, 64, "knn", 128, 4, 0),
+    (20000, 32, 64, "knn", 512, 1, 0),
 ])
 @pytest.mark.parametrize("bits", [32, 16])
 def test_small_batches_equal_large(ctx, cvs, oracle, n, d, degree, kind, itopk, width, iters, bits):
@@ -63,5 +74,29 @@ def test_small_batches_equal_large(ctx, cvs, oracle, n, d, degree, kind, itopk, 
         for q in (1, 128, 129):  # eight and four waves per query
             for got, want, what in zip(search(ctx, cvs, idx, qs[:q], k, knobs), ref, ("ids", "distances", "stats")):
                 np.testing.assert_array_equal(got, want[:q], err_msg=f"{what}, batch of {q}")
+    finally:
+        idx.close()
+
+
+@pytest.mark.parametrize("n,itopk,width", [(262_144, 512, 1), (262_144, 512, 8), (262_144, 65, 2)])
+@pytest.mark.parametrize("bits", [32, 16])
+def test_most_rows(ctx, cvs, n, itopk, width, bits):
+    """The largest visited set of the small-batch kernel (with the longest list
+    and fp16 traversal, more than 64 KiB of LDS) against the same search with
+    its evaluations recorded, which takes one parent at a time."""
+    rng = np.random.default_rng(itopk + width)
+    base = rng.integers(-20, 21, (n, 16)).astype(np.float32)
+    qs = rng.integers(-20, 21, (3, 16)).astype(np.float32)
+    graph = rng.integers(0, n, (n, 64), dtype=np.uint32)
+    idx = ctx.cagra_index(base, graph, cvs.cagra_nav_nodes(n), traversal_bits=bits)
+    try:
+        got = search(ctx, cvs, idx, qs, 10, dict(itopk_size=itopk, search_width=width))
+        nbr, dist = cvs.DeviceArray(ctx, (3, 10), np.uint32), cvs.DeviceArray(ctx, (3, 10), np.float32)
+        st, rec = cvs.DeviceArray(ctx, (3, 2), np.uint32), cvs.DeviceArray(ctx, (3, 64), np.uint32)
+        idx.search_record_async(cvs.DeviceArray.from_host(ctx, qs), 10, nbr, dist, st, rec, itopk_size=itopk,
+                                search_width=width)
+        ctx.synchronize()
+        for g, want, what in zip(got, (nbr, dist, st), ("ids", "distances", "stats")):
+            np.testing.assert_array_equal(g, want.to_host(), err_msg=what)
     finally:
         idx.close()
