@@ -249,22 +249,33 @@ void launch_ks(cvs_context* ctx, const BatchArgs& a, int kp, hipEvent_t e0, hipE
   }
 }
 
+// Fewest ranges of the dataset for lists of kp keys.  A list's final threshold
+// is its kp-th key, and the smallest of them has to lie beyond the merge's
+// R = 2 kp candidates: with one or two ranges it is the kp-th or so key of the
+// whole dataset, and the queries that kp candidates do not certify are
+// re-ranked over every row (131,072 queries, K = 10, 20,000 x 256 in tight
+// clusters: a third of them).  These counts put kp of the 2 kp nearest rows
+// into one range with a probability below 3e-6 (binomial; rows in an order that
+// does not sort them by place).
+int min_ranges(int kp) { return kp <= 16 ? 8 : (kp <= 32 ? 5 : (kp <= 64 ? 4 : 3)); }
+
 }  // namespace
 
-BatchPlan plan_batch_scan(int ks, int64_t q, int64_t n_tiles, int compute_units) {
+BatchPlan plan_batch_scan(int ks, int kp, int64_t q, int64_t n_tiles, int compute_units) {
   BatchPlan p;
   if (ks != 8 && ks != 12 && ks != 16 && ks != 20) return p;
   const int64_t qb = ks <= 8 ? BatchCfg<8>::QB : BatchCfg<12>::QB;
   const int64_t stages = n_tiles / (ks <= 8 ? BatchCfg<8>::TPS : BatchCfg<12>::TPS);
   const int64_t blocks = (q + qb - 1) / qb;
   if (blocks > (int64_t(1) << 20)) return p;
-  // Ranges: one workgroup runs per compute unit, so the fewest ranges (a
-  // list each for the merge to read) that leave at most 1/16 of the last
-  // round of workgroups' units idle, or else the best count.
+  // Ranges: the fewest (each list costs its workgroup a finish and the merge a
+  // read) that leave at most 1/16 of the last round of workgroups' slots idle
+  // (three per compute unit at 8 k-steps, one beyond), or else the best count;
+  // no fewer than the certificate needs (min_ranges).
   const int64_t cu = std::max(1, compute_units) * (ks <= 8 ? 3 : 1);
   const int64_t most = std::min<int64_t>(kBatchMaxRanges, stages);
   double best = 0;
-  for (int64_t g = 1; g <= most; ++g) {
+  for (int64_t g = std::min<int64_t>(min_ranges(kp), most); g <= most; ++g) {
     const int64_t w = g * blocks, rounds = (w + cu - 1) / cu;
     const double eff = double(w) / double(rounds * cu);
     if (eff > best + 1e-9) {

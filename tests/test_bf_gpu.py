@@ -185,6 +185,30 @@ def test_narrow_large_batches(ctx, d, n, q, k):
     assert (nbr[:, m:] == 0xFFFFFFFF).all() and np.isinf(dist[:, m:]).all()
 
 
+@pytest.mark.parametrize("d,q,k", [(256, 131_072, 10), (256, 65_536, 10), (128, 196_608, 24)])
+def test_narrow_batches_of_many_queries(ctx, cvs, d, q, k):
+    """Query counts that fill the chip with one or two ranges of the dataset:
+    there have to be enough candidate lists all the same for the certificate to
+    hold (with one list of 16 keys 29% of these queries at K = 10 fail it, each
+    then re-ranked over every row)."""
+    rng = np.random.default_rng(d + q)
+    n = 20_000
+    centres = rng.standard_normal((64, d)).astype(np.float32)
+    def points(m):
+        x = centres[rng.integers(0, 64, m)] + 0.1 * rng.standard_normal((m, d), dtype=np.float32)
+        return x / np.linalg.norm(x, axis=1, keepdims=True)
+    base, qs = points(n), points(q)
+    ds = ctx.dataset(base)
+    ctx.bf_escalations(reset=True)
+    nbr, dist = ds.bf_search(qs, k)
+    escalated, _ = ctx.bf_escalations(reset=True)
+    assert escalated <= q // 1000
+    some = rng.choice(q, 500, replace=False)
+    want_nbr, want_dist = ds.bf_search(qs[some], k)  # the scan of small batches
+    np.testing.assert_array_equal(nbr[some], want_nbr)
+    np.testing.assert_array_equal(dist[some], want_dist)
+
+
 @pytest.mark.parametrize("q,k", [(2000, 10), (1100, 24)])
 def test_narrow_large_batches_without_allocation(ctx, cvs, q, k):
     """The fixed scratch of the allocation-free call is too small for that
