@@ -1121,29 +1121,25 @@ __global__ __launch_bounds__(256) void bf_merge_filter_kernel(const uint64_t* __
 // ---------------------------------------------------------------------------
 // Merge for kp = 128 (global lists), one workgroup (4 waves) per query; the
 // R = 64 E smallest keys are the candidates.
-//  1. The R-th smallest list minimum bounds the R-th smallest key (R list
-//     minima are R distinct keys): only keys at or below it can be among
-//     the R smallest.  Each wave computes it (a 256-key wave sort) where
-//     there are that many lists.
-//  2. The four waves gather the keys within the bound into LDS, and a radix
-//     select (8 bits a pass, one LDS atomic per key and pass) finds the R-th
+//  1. The smallest list threshold, for the certificate.  (List minima bound
+//     nothing here: fewer lists than R come from every scan, 128 at most.)
+//  2. The four waves gather the listed keys into LDS, and a radix select (8
+//     bits a pass, one LDS atomic per key and pass) finds the R-th
 //     smallest; the keys up to it are the candidates, in any order.  (Sorting
 //     the lists 64 keys at a time into running lists took 22,000 of the
 //     56,000 vector instructions of a query at 25 lists; most of the others
 //     were the re-rank's columns past d = 128.  10,000 queries, K = 100:
 //     1M x 128 1.38 -> 0.89 ms, 1M x 1024 1.85 -> 1.79 ms (re-ranked rows: 10.5 GB).)
-//  2b. More keys within the bound than LDS holds (lists that the sampled
+//  2b. More keys than LDS holds (lists that the sampled
 //     threshold did not shorten): each wave streams a quarter of the lists, 64
-//     keys per row, and merges rows holding a key within its bound into its
-//     running sorted top-64*E, whose R-th key tightens the bound; wave 0
-//     merges the four.
+//     keys per row, and merges rows holding a key up to its bound, the R-th key
+//     of its running sorted top-64*E, into that list; wave 0 merges the four.
 //  3. The candidates are finished (re-ranked, certified) by finish_query.
 // ---------------------------------------------------------------------------
 
-// The need-th smallest (1-based) of the values `v` whose bits above `shift0`
-// + 8 equal those of `pre`, by 8-bit digits from bit shift0 down to 0, over
-// the 256 threads' arrays (count `cnt` of them valid per thread); `need`
-// becomes its rank among the values equal to the result.  s_hist: 256 words.
+// The need-th smallest (1-based) of the 256 threads' values v[i] with ok[i],
+// found by 8-bit digits from the highest down; `need` becomes its rank among
+// the values equal to it.  s_hist: 256 words; s_res: 2.
 template <int M>
 __device__ __forceinline__ uint32_t block_select(const uint32_t (&v)[M], const bool (&ok)[M], int& need,
                                                  uint32_t* s_hist, int* s_res) {
@@ -1194,7 +1190,6 @@ __device__ __forceinline__ uint32_t block_select(const uint32_t (&v)[M], const b
 
 template <int E>
 __global__ __launch_bounds__(256) void bf_merge_kernel(const uint64_t* __restrict__ part,
-                                                       const uint64_t* __restrict__ lmin,
                                                        const float* __restrict__ lcut, int G, int kp, int stride,
                                                        const float* __restrict__ rows, int64_t n, int64_t d,
                                                        const float* __restrict__ queries, int64_t k, Cert cert,
@@ -1214,31 +1209,21 @@ __global__ __launch_bounds__(256) void bf_merge_kernel(const uint64_t* __restric
   constexpr int R = 64 * E;  // candidates re-ranked (>= kp)
   if (tid == 0) s_npass = s_ncid = 0;
 
-  // 1. Bound from the list minima (G <= 256), and the smallest list threshold.
-  // Loads unconditional (index clamped; values past G masked to the sentinel
-  // and +inf by bitwise operations the compiler keeps out of branches): all
-  // eight in flight together.
-  uint64_t mins[4];
+  // 1. The smallest list threshold (G <= 256).  Loads unconditional (index
+  // clamped; values past G masked to +inf by bitwise operations the compiler
+  // keeps out of branches): all four in flight together.
   float cut = INFINITY;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int x = lane + 64 * i;
-    const int64_t xi = q * G + (x < G ? x : G - 1);
-    const uint64_t mv = lmin[xi];
-    const uint32_t cb = __float_as_uint(lcut[xi]);
-    mins[i] = mv | (x < G ? 0ull : kSentinel);
+    const uint32_t cb = __float_as_uint(lcut[q * G + (x < G ? x : G - 1)]);
     cut = fminf(cut, __uint_as_float((cb & (x < G ? 0xffffffffu : 0u)) | (x < G ? 0u : 0x7f800000u)));
   }
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) cut = fminf(cut, xor_lanes_f(cut, o));
-  uint64_t bound = kSentinel;
-  if (G >= R) {
-    wave_sort_e<4>(mins);
-    bound = key_at<4>(mins, R - 1);
-  }
   __syncthreads();  // the counts are zero
 
-  // 2. Gather the keys within the bound.
+  // 2. Gather the keys.
   const uint64_t* src = part + q * int64_t(G) * stride;
   const int total = G * kp;
   const int lkp = __builtin_ctz(kp);  // kp is a power of two
@@ -1253,7 +1238,7 @@ __global__ __launch_bounds__(256) void bf_merge_kernel(const uint64_t* __restric
     uint32_t tot = 0;
 #pragma unroll
     for (int r = 0; r < kBatch; ++r) {
-      m[r] = __ballot(key[r] <= bound && key[r] != kSentinel);
+      m[r] = __ballot(key[r] != kSentinel);
       tot += uint32_t(popc(m[r]));
     }
     if (tot == 0) continue;
@@ -1316,7 +1301,7 @@ __global__ __launch_bounds__(256) void bf_merge_kernel(const uint64_t* __restric
     // 2b. This wave's quarter of the 64-key rows.
     uint64_t (*s_run)[64 * E] = reinterpret_cast<uint64_t (*)[64 * E]>(s_pass);
     __syncthreads();  // s_pass is done with
-    uint64_t run[E];
+    uint64_t run[E], bound = kSentinel;
 #pragma unroll
     for (int e = 0; e < E; ++e) run[e] = kSentinel;
     const int n_rows = (total + 63) / 64;
@@ -1670,8 +1655,7 @@ void bf_launch(cvs_context* ctx, const cvs_dataset* ds, const BfPlan& p, const f
                           ds->d, queries, k, cert, nbr, dist);
   else
     hipExtLaunchKernelGGL(bf_merge_kernel<4>, dim3(unsigned(q)), dim3(kThreads), 0, ctx->stream, t3.start, t3.stop,
-                          0, static_cast<const uint64_t*>(part), static_cast<const uint64_t*>(lmin),
-                          static_cast<const float*>(lcut), G, kp, p.stride, static_cast<const float*>(ds->rows), ds->n,
+                          0, static_cast<const uint64_t*>(part), static_cast<const float*>(lcut), G, kp, p.stride, static_cast<const float*>(ds->rows), ds->n,
                           ds->d, queries, k, cert, nbr, dist);
   after_launch("bf_merge_kernel");
 }
