@@ -951,17 +951,20 @@ __device__ void finish_query(const uint32_t* s_cid, int R, float t_cert, float t
 // Merge for kp <= 64, one workgroup (4 waves) per query.
 //  1. The R-th smallest list minimum (R = min(2 kp, 64 E)) bounds the R-th
 //     smallest key (R list minima are R distinct keys): only keys at or
-//     below it can be among the R smallest.  Wave 0 computes it (a 256-key
-//     wave sort) and the smallest list threshold T* while every wave's first
-//     batch of keys is already in flight.
-//  2. A key within the bound comes from one of the R lists whose minimum is
-//     within it, so at most R * kp keys pass.  The four waves stream all
-//     G * kp keys and append the passing ones to an LDS buffer of that size
-//     (one atomic per wave and batch).
+//     below it can be among the R smallest.  Wave 0 computes it (or, from a
+//     smaller sort, a slightly looser bound) and the smallest list threshold
+//     T* while every wave's first batch of keys is already in flight.
+//  2. The four waves stream all G * kp keys and append those within the bound
+//     to an LDS buffer (one atomic per wave and batch).  For kp <= 32 at most
+//     128 lists have a minimum within the bound (a lane looks after four, and
+//     32 lanes' worth of minima lie within it), which the buffer holds.  For
+//     kp = 64 more keys than it holds may pass; step 3 says what happens then.
 //  3. Wave 0 sorts the passing keys 64 at a time and merges them into its
 //     running sorted top-64 E; its first R ids are finished (re-ranked,
 //     certified) by finish_query.
 // ---------------------------------------------------------------------------
+constexpr int kFilterMaxKeys = 64 * 64;
+
 template <int E>
 __global__ __launch_bounds__(256) void bf_merge_filter_kernel(const uint64_t* __restrict__ part,
                                                               const uint64_t* __restrict__ lmin,
@@ -971,8 +974,8 @@ __global__ __launch_bounds__(256) void bf_merge_filter_kernel(const uint64_t* __
                                                               const float* __restrict__ queries, int64_t k,
                                                               Cert cert, uint32_t* __restrict__ out_nbr,
                                                               float* __restrict__ out_dist) {
-  constexpr int kBatch = 16;        // keys per thread and batch
-  constexpr int kMaxPass = 64 * 64; // passing keys held in LDS
+  constexpr int kBatch = 16;                // keys per thread and batch
+  constexpr int kMaxPass = kFilterMaxKeys;  // passing keys held in LDS
   __shared__ uint64_t s_pass[kMaxPass];
   __shared__ uint32_t s_npass;
   __shared__ uint64_t s_bound, s_keyr;
@@ -1087,7 +1090,7 @@ __global__ __launch_bounds__(256) void bf_merge_filter_kernel(const uint64_t* __
   __syncthreads();
 
   // 3. Wave 0: top-R of the passing keys.  Should more keys pass than LDS
-  // holds (not seen in practice), the candidates are not known to be the R
+  // holds, the candidates are not known to be the R
   // smallest: the certificate is then made to fail, and the escalation
   // re-ranks from the lists afresh.
   if (wave == 0) {
@@ -1119,8 +1122,9 @@ __global__ __launch_bounds__(256) void bf_merge_filter_kernel(const uint64_t* __
 }
 
 // ---------------------------------------------------------------------------
-// Merge for kp = 128 (global lists), one workgroup (4 waves) per query; the
-// R = 64 E smallest keys are the candidates.
+// Merge for kp = 128 (E = 4), and for more lists of kp = 64 than the filter
+// merge has room for (E = 2); one workgroup (4 waves) per query.  The R = 64 E
+// smallest keys are the candidates.
 //  1. The smallest list threshold, for the certificate.  (List minima bound
 //     nothing here: fewer lists than R come from every scan, 128 at most.)
 //  2. The four waves gather the listed keys into LDS, and a radix select (8
@@ -1643,11 +1647,20 @@ void bf_launch(cvs_context* ctx, const cvs_dataset* ds, const BfPlan& p, const f
   // between the k-th result and the last candidate is what lets the
   // certificate pass: on the benchmark's distribution at N = 1M, 16
   // candidates for k = 10 or 128 for k = 100 leave most queries uncertified.
+  //
+  // kp = 64: the large-batch scan over narrow rows may give up to 128 lists,
+  // too few for a bound on their keys and with more keys than the filter
+  // merge's buffer (from about 20 million rows on, or where the sample misses
+  // the nearest rows): bf_merge_kernel has a way for those.
   if (kp <= 32)
     hipExtLaunchKernelGGL(bf_merge_filter_kernel<1>, dim3(unsigned(q)), dim3(kThreads), 0, ctx->stream, t3.start,
                           t3.stop, 0, static_cast<const uint64_t*>(part), static_cast<const uint64_t*>(lmin),
                           static_cast<const float*>(lcut), G, kp, p.stride, static_cast<const float*>(ds->rows), ds->n,
                           ds->d, queries, k, cert, nbr, dist);
+  else if (kp == 64 && p.batch && G * kp > kFilterMaxKeys)
+    hipExtLaunchKernelGGL(bf_merge_kernel<2>, dim3(unsigned(q)), dim3(kThreads), 0, ctx->stream, t3.start, t3.stop,
+                          0, static_cast<const uint64_t*>(part), static_cast<const float*>(lcut), G, kp, p.stride,
+                          static_cast<const float*>(ds->rows), ds->n, ds->d, queries, k, cert, nbr, dist);
   else if (kp <= 64)
     hipExtLaunchKernelGGL(bf_merge_filter_kernel<2>, dim3(unsigned(q)), dim3(kThreads), 0, ctx->stream, t3.start,
                           t3.stop, 0, static_cast<const uint64_t*>(part), static_cast<const uint64_t*>(lmin),
@@ -1655,8 +1668,8 @@ void bf_launch(cvs_context* ctx, const cvs_dataset* ds, const BfPlan& p, const f
                           ds->d, queries, k, cert, nbr, dist);
   else
     hipExtLaunchKernelGGL(bf_merge_kernel<4>, dim3(unsigned(q)), dim3(kThreads), 0, ctx->stream, t3.start, t3.stop,
-                          0, static_cast<const uint64_t*>(part), static_cast<const float*>(lcut), G, kp, p.stride, static_cast<const float*>(ds->rows), ds->n,
-                          ds->d, queries, k, cert, nbr, dist);
+                          0, static_cast<const uint64_t*>(part), static_cast<const float*>(lcut), G, kp, p.stride,
+                          static_cast<const float*>(ds->rows), ds->n, ds->d, queries, k, cert, nbr, dist);
   after_launch("bf_merge_kernel");
 }
 

@@ -209,6 +209,26 @@ def test_narrow_batches_of_many_queries(ctx, cvs, d, q, k):
     np.testing.assert_array_equal(dist[some], want_dist)
 
 
+@pytest.mark.parametrize("d,q,k", [(128, 1100, 48), (200, 1100, 25), (128, 1100, 24), (128, 2900, 48)])
+def test_narrow_large_batches_with_long_lists(ctx, d, q, k):
+    """Full candidate lists, 64 (the last row) to 128 a query: the nearest rows
+    lie where the threshold sample does not look (it takes every third unit of
+    256 rows, or 128 beyond 128 columns), so that two thirds of the rows pass its threshold.  No query may
+    need an escalation for it."""
+    rng = np.random.default_rng(d + q + k)
+    n = 100_000
+    base = rng.standard_normal((n, d), dtype=np.float32)
+    base[np.arange(n) // (256 if d <= 128 else 128) % 3 == 0] *= 1.6
+    qs = rng.standard_normal((q, d), dtype=np.float32)
+    ds = ctx.dataset(base)
+    ctx.bf_escalations(reset=True)
+    nbr, dist = ds.bf_search(qs, k)
+    assert ctx.bf_escalations(reset=True)[0] == 0
+    want_nbr, want_dist = ds.bf_search(qs[:500], k)  # the scan of small batches
+    np.testing.assert_array_equal(nbr[:500], want_nbr)
+    np.testing.assert_array_equal(dist[:500], want_dist)
+
+
 @pytest.mark.parametrize("q,k", [(2000, 10), (1100, 24)])
 def test_narrow_large_batches_without_allocation(ctx, cvs, q, k):
     """The fixed scratch of the allocation-free call is too small for that
