@@ -259,11 +259,28 @@ void launch_ks(cvs_context* ctx, const BatchArgs& a, int kp, hipEvent_t e0, hipE
 // does not sort them by place).
 int min_ranges(int kp) { return kp <= 16 ? 8 : (kp <= 32 ? 5 : (kp <= 64 ? 4 : 3)); }
 
+// Whether this scan is the faster one (the other: the streaming scan, or for kp
+// = 128 the register-blocked one, slower at all but one of 156 sizes).  Its
+// workgroups finish 64 lists a wave however few rows they have seen, which
+// small calls do not make up for.  Streaming scan against this one, K = 10, d =
+// 96 / 256 / 320 (us, whole calls): 20,000 rows, 2,000 queries 135 / 164 / 190
+// against 145 / 179 / 212, 4,000 queries 236 / 297 / 337 against 221 / 285 /
+// 336; 40,000 rows, 1,100 queries 149 / 193 / 194 against 139 / 172 / 185.  The
+// line lies lower for K = 24, and for K = 48 only calls of few thousand rows
+// lie below it.
+bool pays(int ks, int kp, int64_t q, int64_t n) {
+  if (kp > 64) return true;
+  if (kp == 64) return n >= 5000 || q >= 3000 || (n < 1500 && ks < 20);
+  const double t = kp <= 16 ? 5500.0 : 4000.0;
+  return n >= 4000 ? double(q) >= t * (1.0 - double(n) / 48000.0) : n >= 2000 && double(q) >= 1.5 * t;
+}
+
 }  // namespace
 
-BatchPlan plan_batch_scan(int ks, int kp, int64_t q, int64_t n_tiles, int compute_units) {
+BatchPlan plan_batch_scan(int ks, int kp, int64_t q, int64_t n, int64_t n_tiles, int compute_units) {
   BatchPlan p;
   if (ks != 8 && ks != 12 && ks != 16 && ks != 20) return p;
+  if (!pays(ks, kp, q, n)) return p;
   const int64_t qb = ks <= 8 ? BatchCfg<8>::QB : BatchCfg<12>::QB;
   const int64_t stages = n_tiles / (ks <= 8 ? BatchCfg<8>::TPS : BatchCfg<12>::TPS);
   const int64_t blocks = (q + qb - 1) / qb;

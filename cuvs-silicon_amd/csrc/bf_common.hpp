@@ -392,11 +392,11 @@ struct BatchArgs {
   int n_qblocks;
 };
 struct BatchPlan {
-  bool ok = false;      // false: not a padded dimension it handles
+  bool ok = false;      // false: not a shape it handles, or not the faster scan there
   int n_ranges = 0;     // candidate lists per query
   int n_qblocks = 0;
 };
-BatchPlan plan_batch_scan(int ks, int kp, int64_t q, int64_t n_tiles, int compute_units);
+BatchPlan plan_batch_scan(int ks, int kp, int64_t q, int64_t n, int64_t n_tiles, int compute_units);
 void launch_batch_scan(cvs_context* ctx, const BatchArgs& args, int ks, int kp, hipEvent_t e0, hipEvent_t e1);
 
 }  // namespace bf

@@ -1473,7 +1473,7 @@ BfPlan plan_bf(cvs_context* ctx, const cvs_dataset* ds, const float* queries, in
   // with kp = 128 the register-blocked scan: persistent workgroups over
   // (query block, row block) units, n_lists lists per query.
   BatchPlan bp;
-  if (p.large_batch && batch) bp = plan_batch_scan(p.ks, p.kp, q, ds->n_tiles, ctx->compute_units);
+  if (p.large_batch && batch) bp = plan_batch_scan(p.ks, p.kp, q, ds->n, ds->n_tiles, ctx->compute_units);
   if (bp.ok) {
     p.batch = true;
     p.batch_qblocks = bp.n_qblocks;
