@@ -29,8 +29,9 @@
 //    before the sort.
 //  - waves per query: 2 for large batches; 4 or 8 when the batch is small
 //    and each query's chain of dependent gathers is the latency (Q = 1).
-//    Most of those small batches run cagra_ahead_kernel, which shortens that
-//    chain: the rows of several parents gathered in one step.
+//    With long lists or wide searches (ahead_from) those small batches run
+//    cagra_ahead_kernel, which shortens that chain: the rows of several
+//    parents gathered in one step.
 //
 // Iteration: pick the first `width` unexpanded entries of the list as
 // parents, mark them, evaluate their neighbours.  Stop when the list holds no
@@ -1390,6 +1391,40 @@ int ceil_log2(int64_t v) {
   return b;
 }
 
+// Shortest list with which cagra_ahead_kernel is faster than
+// cagra_search_kernel (4 or 8 waves per query, up to 512 queries).  It saves
+// the other kernel's steps, one per iteration, where most expansions are of
+// entries that have been in the list for some time, and loses the rows that it
+// gathers in vain.  Three things decide, all measured on both kernels at 15,000
+// to 100,000 rows, d = 96 to 1,024, degree 16 to 64, fp32 and fp16 (ratios of
+// the times, other kernel / this one; fp32, 100,000 x 768, degree 64 unless
+// said otherwise):
+//  - the list: width 1, Q = 1, itopk 48 0.99, 64 1.11, 128 1.50, 512 2.07.
+//  - queries that share the caches' bandwidth: itopk 64, Q = 60 1.03 (15,000 x
+//    256, Q = 30: 0.76), 128 0.87; with four waves (beyond 128 queries) Q = 300,
+//    itopk 128 0.88, 256 1.16, 512 1.62.  A wide search gathers little in vain:
+//    width 8, itopk 65, Q = 128 1.33, Q = 300 1.10.
+//  - iterations of several parents with one chunk of 64 candidates: degree 32,
+//    width 2, Q = 1, itopk 64 0.72, 128 0.90, 256 1.18, 512 1.40; degree 16,
+//    width 4, itopk 512 0.91.
+// Below the line the two differ little or the other kernel is faster.  A batch
+// takes as long as its longest walk, so single ones lie on the other side
+// (30,000 x 512, width 1, itopk 96 to 192, Q = 60, one walk of 384 nodes: 0.84).
+int64_t ahead_from(int waves, int64_t q, int64_t n, int64_t width, int64_t degree) {
+  const double parents = double(width) / double((width * degree + 63) / 64);  // per chunk
+  if (parents > 2.0) return CVS_CAGRA_MAX_ITOPK + 1;
+  double least;
+  if (waves == 8) {
+    const bool few = q <= 8 || (q <= 64 && n >= 32'768);
+    least = width == 1 ? (few ? 64.0 : 96.0) * std::max(1.0, 32.0 / double(degree))
+                       : (width <= 4 ? 64.0 : (width <= 6 ? 48.0 : 33.0));
+  } else {
+    least = width == 1 ? (q <= 384 ? 256.0 : 512.0)
+                       : (width <= 3 ? 256.0 : (width == 4 ? 192.0 : (width <= 6 ? 128.0 : 65.0)));
+  }
+  return int64_t(std::min(512.0, least * parents * parents));
+}
+
 void cagra_search_device(cvs_context* ctx, const cvs_cagra_index* idx, const float* queries,
                          int64_t q, int64_t k, uint32_t itopk_size, uint32_t search_width,
                          uint32_t max_iterations, uint32_t* nbr, float* dist, uint32_t* stats, int teams = 1,
@@ -1431,20 +1466,13 @@ void cagra_search_device(cvs_context* ctx, const cvs_cagra_index* idx, const flo
   const size_t visit_words = use_bitmap ? size_t(bitmap_words) : (size_t(1) << hash_bits);
   // (The visited set's words hold the query first, see cagra_search_kernel.)
   // Small batches gather for several entries at a time (cagra_ahead_kernel)
-  // where that is the faster way.  It pays once the list is long enough that
-  // most expansions are of entries already in it: at N=100K D=1024 fp32,
-  // without and with it, itopk 32 Q=1 125 / 147 us (not taken), 64 Q=1 213 /
-  // 185, Q=128 265 / 246, 128 Q=1 414 / 244, 512 Q=100 1611 / 806.  With four
-  // waves (129 to 512 queries) compute units are shared, and the rows that
-  // are gathered in vain cost more: itopk 64 Q=300 307 / 359 (not taken), 128
-  // Q=200 500 / 435, Q=500 545 / 534, 512 Q=500 1534 / 1077.  Teams walk from
-  // scattered seeds with short lists (8 teams x 32, Q=1: 123 / 175; 4 x 64:
-  // 213 / 250; not taken), and beyond 512 workgroups it is slower at any
-  // itopk (512 Q=1,000: 1737 / 2038).  Six entries are best for one key per
-  // lane (4: 196, 8: 192 us at Q=1), eight for longer lists.
+  // where that is the faster way (ahead_from).  Teams walk from scattered seeds
+  // with short lists (8 teams x 32, Q=1: 123 us without it, 175 with it; 4 x 64:
+  // 213 / 250; not taken).  Six entries are best for one key per lane (4: 196,
+  // 8: 192 us at Q=1), eight for longer lists.
   int ahead = 0;
   if (waves >= 4 && !big && use_bitmap && idx->degree <= 64 && width <= kAhead && teams == 1 && !record &&
-      itopk > (waves == 8 ? 32 : 64))
+      itopk >= ahead_from(waves, q, idx->n, width, idx->degree))
     ahead = std::max(itopk > 64 ? kAhead : 6, int(width));
   const bool f16 = idx->traversal_bits == 16;
   size_t lds = (big ? visit_words : std::max<size_t>(visit_words, kBigDim)) * 4 + (64 + 64 + CVS_CAGRA_MAX_WIDTH + 8) * 4 +

@@ -46,6 +46,14 @@ def search(ctx, cvs, idx, qs, k, knobs):
     (5000, 1024, 64, "knn", 10, 1, 0),       # a list shorter than the parents gathered ahead
     (3000, 128, 32, "random", 300, 4, 7),    # cut off by max_iterations
     (1, 16, 1, "random", 32, 1, 0),
+    # Narrow iterations, part-filled chunks, too few rows, cut off, with lists
+    # long enough for the kernel.
+    (2049, 64, 48, "random", 65, 8, 0),
+    (2049, 64, 33, "holes", 192, 3, 0),
+    (3000, 100, 32, "knn", 256, 2, 0),
+    (40, 24, 33, "random", 512, 2, 0),
+    (3000, 128, 64, "random", 300, 4, 7),
+    (1, 16, 1, "random", 512, 1, 0),
     # Hundreds of new keys in one step, again and again: the pool's buffer has
     # to hold up to 999 keys.  Every list length; wide steps and runs of single
     # parents.
