@@ -7,6 +7,8 @@
 - test_api_gpu (GPU): the FAISS v1.8 adapter flow and known answers, the
   dispatch test with its exact answers, the exact route and the brute_force
   namespace, build -> save -> load -> search recall.
+- test_descent (GPU): nn-descent's iterations over new pairs against
+  iterations over every pair, list by list (the kernel's source compiled in).
 - test_loaders (no GPU): fvecs/ivecs and Cohere .bin readers.
 - asan_test_api_cpu, asan_test_loaders (no GPU): the two above with the
   library's host sources compiled in under AddressSanitizer (leaks
@@ -46,6 +48,11 @@ def test_api_cpu(tmp_path):
 @pytest.mark.gpu
 def test_api_gpu(tmp_path):
     run("test_api_gpu", str(tmp_path))
+
+
+@pytest.mark.gpu
+def test_descent():
+    run("test_descent")
 
 
 def test_loaders(tmp_path):
