@@ -1,5 +1,6 @@
 // Exact-search scan of large query batches over narrow rows (gfx950): 8 to 20
-// k-steps per tile (d from 65 to 320), more than 1,024 queries.
+// k-steps per tile (d from 65 to 320), more than 1,024 queries, but for small
+// calls (pays, below).
 //
 // With few k-steps per row tile the two other scans spend their time beside
 // the matrix cores: the streaming scan (bf_search.hip) reads one LDS fragment
@@ -22,9 +23,9 @@
 //    smallest keys.
 //
 // 10,000 queries, K = 100, 1M x 128: the register-blocked scan took 6.71 ms,
-// this one 3.02 (2.56 TFLOP: 0.34 of the 2.5 PFLOP/s peak; MFMA busy 0.37 of
-// the cycles, other vector instructions 0.27).  What is left is latency that
-// three waves do not hide.  Four query tiles per wave at two waves per SIMD
+// this one 3.02 to 3.2 (2.56 TFLOP: 0.34 of the 2.5 PFLOP/s peak; the SIMDs'
+// cycles: MFMA busy 0.42, other vector instructions 0.35).  What is left is
+// latency that three waves do not hide: they wait 0.46 of their cycles.  Four query tiles per wave at two waves per SIMD
 // took 3.28 ms (4.25 with the rows staged through registers, which spilled),
 // and left small batches short of workgroups: 1,500 queries K = 10 1M x 128
 // 717 us, 575 now, 1,314 as the streaming scan.
@@ -35,7 +36,6 @@
 namespace cvs {
 namespace bf {
 namespace {
-
 
 // Smallest of three; skips NaN, which passes no threshold either.  (fminf
 // costs a canonicalising instruction per operand.)

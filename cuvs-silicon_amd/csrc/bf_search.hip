@@ -13,9 +13,8 @@
 //  sample   the scan kernel over an evenly strided sample of 16,384 rows
 //           (65,536 for other large batches, 32,768 when one of the
 //           large-batch scans of bf_gemm.hip and bf_batch.hip follows); each
-//           lane keeps the minimum distance
-//           of the rows it sees, so every (query, workgroup, half-wave)
-//           yields one minimum.
+//           lane keeps the minimum distance of the rows it sees, so every
+//           (query, workgroup, half-wave) yields one minimum.
 //  select   per query (one wave), the r-th smallest of those minima (or, for
 //           small batches, of the lanes' minima of them), T0.  The r
 //           smallest minima are r distinct dataset rows, so at least r
@@ -37,13 +36,13 @@
 //           keys (ballot radix select), lowering the threshold.  Lists of
 //           kp <= 64 live in LDS, kp = 128 lists in global memory.  Each list
 //           ends with its smallest key published for the merge.
-//  merge    one workgroup per query: the R-th smallest list minimum bounds
-//           the R-th smallest key (R = 2 kp, at most 256).  For kp <= 64 every
-//           key within it is gathered into LDS and one wave keeps the R
-//           smallest; for kp = 128 a radix select finds the R-th.  The R
-//           candidates
-//           are re-ranked with exact fp32 distances from the fp32 rows,
-//           sorted by (distance, id), certified against the fp16 error bound
+//  merge    one workgroup per query: the R smallest listed keys (R = 2 kp, at
+//           most 256).  For kp <= 64 the R-th smallest list minimum bounds
+//           them, every key within it is gathered into LDS, and one wave keeps
+//           the R smallest; for kp = 128 (and many lists of 64) all are
+//           gathered and a radix select finds the R-th.  The R candidates are
+//           re-ranked with exact fp32 distances from the fp32 rows, sorted by
+//           (distance, id), certified against the fp16 error bound
 //           (bf_common.hpp, Cert; a query that fails is re-ranked over more
 //           rows), and k results written, padded with UINT32_MAX / +inf
 //           (src/cagra.cpp:240-251).

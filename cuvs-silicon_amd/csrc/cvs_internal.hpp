@@ -191,8 +191,8 @@ constexpr int kNormSlack = 256;  // floats allocated past the last tile's norms
 // (bf_search.hip, Cfg): a third, or less, of steps between them, so that a
 // scan bound by its bytes reads little padding.  With only powers of two, d =
 // 768 and 771 streamed 1024 columns: one host query to 100,000 x 768 took 127
-// us, 115 now; 37 queries to 499,979 x 771 200 us, 183 now.  Beyond, multiples of 64 (only the keys-matrix path reads those, four
-// k-steps at a time).
+// us, 115 now; 37 queries to 499,979 x 771 200 us, 183 now.  Beyond, multiples
+// of 64 (only the keys-matrix path reads those, four k-steps at a time).
 inline int64_t padded_dim(int64_t d) {
   if (d > 1024) return (d + 63) / 64 * 64;
   for (const int ks : {2, 4, 8, 12, 16, 20, 24, 28, 32, 40, 48, 56})

@@ -282,8 +282,8 @@ def test_every_padded_dimension(ctx, d, n, q, k):
     (12000, 512, 1100, 40),   # range-major pipelined scan (32 k-steps), kp = 64 LDS lists
     (7000, 384, 1100, 100),   # 24 k-steps
     (5000, 640, 1030, 50),    # 40 k-steps; the last 512-query block holds one 32-query tile
-    (9000, 768, 1200, 112),   # d 768 padded to 1024, largest k
-    (3000, 896, 2100, 77),    # d 896 padded to 1024, 5 query blocks
+    (9000, 768, 1200, 112),   # 48 k-steps, largest k
+    (3000, 896, 2100, 77),    # 56 k-steps, 5 query blocks
 ])
 def test_large_batches(ctx, oracle, n, d, q, k):
     rng = np.random.default_rng(q + k)
