@@ -266,12 +266,14 @@ int min_ranges(int kp) { return kp <= 16 ? 8 : (kp <= 32 ? 5 : (kp <= 64 ? 4 : 3
 // 96 / 256 / 320 (us, whole calls): 20,000 rows, 2,000 queries 135 / 164 / 190
 // against 145 / 179 / 212, 4,000 queries 236 / 297 / 337 against 221 / 285 /
 // 336; 40,000 rows, 1,100 queries 149 / 193 / 194 against 139 / 172 / 185.  The
-// line lies lower for K = 24, and for K = 48 only calls of few thousand rows
-// lie below it.
+// line lies lower for K = 24 (10,000 rows, 3,000 queries, d = 96 / 256: 214 /
+// 227 against 192 / 219), and for K = 48 only calls whose rows fill most of one
+// unit of 2,048 lie below it (2,000 rows, 1,100 queries: 1.05 to 1.2x slower
+// here; 1,500 rows, up to 16 k-steps: 1.3 to 2.5x faster).
 bool pays(int ks, int kp, int64_t q, int64_t n) {
   if (kp > 64) return true;
-  if (kp == 64) return n >= 5000 || q >= 3000 || (n < 1500 && ks < 20);
-  const double t = kp <= 16 ? 5500.0 : 4000.0;
+  if (kp == 64) return q >= 3000 || n > 2048 || (n <= 1700 && ks < 20);
+  const double t = kp <= 16 ? 5500.0 : 3500.0;
   return n >= 4000 ? double(q) >= t * (1.0 - double(n) / 48000.0) : n >= 2000 && double(q) >= 1.5 * t;
 }
 

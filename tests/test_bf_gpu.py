@@ -167,7 +167,7 @@ def test_merge_of_long_lists(ctx, d, copies, k):
     (30000, 1030, 112),
     (40001, 1025, 10), (4100, 5201, 7), (2000, 8250, 3),  # 16-key lists: fewer rows or queries take the other scan
     (36001, 1030, 24), (2100, 6001, 20),                  # 32-key lists
-    (5000, 1100, 48), (1500, 3000, 30), (1499, 1100, 48),  # 64-key lists
+    (2500, 1100, 48), (1500, 3000, 30), (1499, 1100, 48),  # 64-key lists
 ])
 def test_narrow_large_batches(ctx, d, n, q, k):
     """The large-batch scan over 8 to 20 k-steps, every list geometry.  Rows
